@@ -47,13 +47,20 @@ def rms_norm(x: torch.Tensor, weight: torch.Tensor, eps: float) -> torch.Tensor:
 
 
 # bf16 projections of at most this many rows run on specdec_linear (one
-# pass over the weight with every load in flight; a row's bits do not
-# depend on the other rows), reading the weight's tiled copy where the
-# layer has one (any inner size up to 8192) and the row-major weight up to
-# LINEAR_K; more rows (prompts) run on torch's GEMM.  SPECDEC_TORCH_PROJECTIONS=1
-# (or LINEAR_KERNEL = False before a model's graphs are captured) keeps
-# every projection on torch.
-LINEAR_ROWS, LINEAR_K = 16, 2048
+# pass over the weight; a row's bits do not depend on the other rows): up to
+# LINEAR_ROWS rows with the weight's tiled copy (any inner size up to 8192),
+# up to LINEAR_ROWS_PLAIN rows and LINEAR_K with a row-major weight; more rows
+# (prompts) run on torch's GEMM.  At 40 rows the 1.7B's qkv / o / down take
+# 10.0 / 6.4 / 14.5 us against 13.0 / 11.2 / 14.1 us on torch, at 64 rows 10.6 /
+# 7.2 / 16.1 against 12.8 / 11.7 / 22.6 us; the draft's 3.1 / 3.5 / 4.5 against
+# 6 / 6 / 7 us.  SPECDEC_TORCH_PROJECTIONS=1 (or LINEAR_KERNEL = False before a
+# model's graphs are captured) keeps every projection on torch.
+LINEAR_ROWS, LINEAR_ROWS_PLAIN, LINEAR_K = ops.LINEAR_ROWS, 16, 2048
+# The gate/up form of a wide weight: every workgroup repeats the rows' norm
+# scales, and past this many rows torch's GEMM and rms_silu_mul are faster (the
+# 1.7B, 16384 x 2048: 20.1 against 21.7 us at 40 rows, 23.5 against 21.0 us at
+# 64; the draft, 3072 x 576: 6.2 against 8.8 us at 64).
+SILU_ROWS_WIDE, SILU_WIDE = 48, 1 << 24
 LINEAR_KERNEL = os.environ.get("SPECDEC_TORCH_PROJECTIONS", "0") != "1"
 
 
@@ -66,9 +73,17 @@ def _linear_weight(x: torch.Tensor, w: torch.Tensor, wt: torch.Tensor | None = N
         return None
     if wt is not None and ops.linear_fits(x, wt):
         return wt
-    if k <= LINEAR_K and ops.linear_fits(x, w):
+    if x.numel() <= LINEAR_ROWS_PLAIN * k and k <= LINEAR_K and ops.linear_fits(x, w):
         return w
     return None
+
+
+def _silu_weight(x: torch.Tensor, w: torch.Tensor, wt: torch.Tensor | None) -> torch.Tensor | None:
+    """The gate/up weight specdec_linear_silu reads, or None when the call
+    runs as torch's GEMM and rms_silu_mul."""
+    if w.numel() > SILU_WIDE and x.numel() > SILU_ROWS_WIDE * w.shape[-1]:
+        return None
+    return _linear_weight(x, w, wt)
 
 
 def _project(x: torch.Tensor, w: torch.Tensor, gemv: bool, wt: torch.Tensor | None = None) -> torch.Tensor:
@@ -151,7 +166,7 @@ def forward_core(llama: Llama, cache: KVCache, meta: torch.Tensor, ids: torch.Te
                                      h, hk, d, cache.block_size, llama.scaling, max_kv_len, attn, attn.stride(1),
                                      workspace, split_tokens, norm_of=hidden if in_attn else None, eps=eps)
             _project_add(hidden, attn, layer.wo, gemv, layer.wo_t)
-        gw = _linear_weight(hidden, layer.wgu, layer.wgu_t)
+        gw = _silu_weight(hidden, layer.wgu, layer.wgu_t)
         if gw is not None:  # gate/up and the MLP's norm + activation in one launch
             ops.linear_silu(hidden, gw, hidden, act, eps)
         else:
