@@ -1347,240 +1347,251 @@ __global__ __launch_bounds__(kWave) void attention_decode_parts_kernel(AttnArgs 
 // ------------------------------------------------------------- prefill ----
 // Wide bf16 calls (more than kStage new tokens per row: a prompt), with the
 // new K/V already in the pools (rope_append ran first, or the caller wrote
-// them).  One 8-wave workgroup per (row, kv head, eight consecutive 16-row
-// query tiles); each wave owns one tile.  The workgroup walks its keys in
-// 128-token stages: each stage's K and V tiles (8 pool tiles of 16 tokens,
-// 32 KB) are staged into LDS once, with coalesced 16-byte loads issued two
-// stages ahead (three LDS buffers: a stage's loads have two stages' compute
-// to arrive in), two 64-token steps per stage; every wave reads its MFMA
-// operands from LDS, and a wave whose queries end before a step skips it.  Online softmax in registers, then O / l.  No split partials,
-// no cross-wave fold.  Per step and wave the arithmetic is the decode
-// kernel's (K rows permuted so P^T comes out of the S^T accumulators); the
-// fold order differs from the split kernels', so prefill rows need not equal
-// the bits a decode step of the same token would get (nothing compares
-// them: every path prefills with this kernel).
-constexpr int kPrefillTiles = 8;                     // query tiles (waves) per workgroup
-constexpr int kPrefillThreads = kPrefillTiles * kWave;
-constexpr int kPKStride = kD + 8;                    // bf16 per staged K row (token): 144 bytes
-constexpr int kPVStride = 16 + 8;                    // bf16 per staged V row (dim of a 16-token group): 48 bytes
-constexpr int kPStage = 128;                         // tokens per staged stage
-constexpr int kPGroups = kPStage / 16;               // 16-token groups per stage
-constexpr int kPKElems = kPStage * kPKStride;        // one stage's K
-constexpr int kPVElems = kPGroups * kD * kPVStride;  // one stage's V: [group][dim][token]
-constexpr int kPUnits = 2 * kPGroups * 128 / kPrefillThreads;  // 16-byte staging units per thread
+// them).  Bound by the softmax's vector arithmetic (about 30 cycles a score
+// and wave) with the MFMAs beside it, so a wave takes 32 query rows on
+// v_mfma_f32_32x32x16_bf16: half the LDS operand reads per score of 16-row
+// tiles, the row maximum one lane exchange away, and no rescale of O in steps
+// where no row's maximum grew.
+//   S^T[key, query] = K . Q^T    lane (q = lane % 32, h = lane / 32) holds 16
+//                                keys of query q
+//   O^T[dim, query] += V^T . P^T
+// K rows are read permuted (key_of_row) so that a lane's eight S^T values of
+// a 16-key group are keys 8h .. 8h+7, which is the P^T operand.  One workgroup
+// of four waves per (row, kv head, 128 query rows); it walks its causal keys in
+// 64-key stages, staged into LDS once for all waves (two buffers), with the
+// loads issued two stages ahead.  The blocks with the most keys start first.
+// A wave's arithmetic depends on its rows alone: a prompt's rows have the same
+// bits in any batch.  The fold order
+// differs from the split kernels', so prefill rows need not equal the bits a
+// decode step of the same token would get.
+// MI355X, 32 heads: 4 x 1024 tokens 34 us (470 TFLOP/s), 1 x 4096 tokens 98 us
+// (700); a kernel of 16-row waves took 100 and 361.
+typedef __attribute__((ext_vector_type(16))) float f32x16;
+constexpr int kPRows = 32;                        // query rows of a wave
+constexpr int kPWaves = 4, kPThreads = kPWaves * kWave;
+constexpr int kPBlock = kPRows * kPWaves;         // query rows of a workgroup
+constexpr int kPStage = 64;                       // keys of a stage
+constexpr int kPElems = kPStage * kD;             // one stage's K, or its V
+constexpr int kPUnits = 2 * kPElems * 2 / 16 / kPThreads;  // 16-byte staging units per thread: K, then V
+
+// The lanes' other half-wave's value.
+__device__ __forceinline__ float other_half(float v) {
+  const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+  return __uint_as_float((threadIdx.x & 32) ? r[0] : r[1]);
+}
 
 template <int MODE>
-__global__ __launch_bounds__(kPrefillThreads) void attention_prefill_kernel(AttnArgs a) {
-  __shared__ __align__(16) unsigned short s_k[3][kPKElems];
-  __shared__ __align__(16) unsigned short s_v[3][kPVElems];
+__global__ __launch_bounds__(kPThreads) __attribute__((amdgpu_waves_per_eu(3))) void attention_prefill_kernel(
+    AttnArgs a) {
   typedef unsigned short u16;
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const int g = lane >> 4, c = lane & 15;
-  const int nqb = (a.n_qtiles + kPrefillTiles - 1) / kPrefillTiles;
-  const int qb = blockIdx.x % nqb, bh = blockIdx.x / nqb;
-  const int qt = qb * kPrefillTiles + wave;
-  // this wave's tile; a wave without one (past the tiles, or rows past the
-  // row's new tokens) still stages and meets the barriers
-  TileInfo ti;
-  const bool live = qt < a.n_qtiles && tile_info_at(a, bh * a.n_qtiles + qt, ti, /*any_split=*/true);
-  if (!live && qt < a.n_qtiles && ti.overflow && ti.qt * kRows + c < ti.nrows) {
-    // beyond max_kv_len: NaN rows, as the other kernels
-    const int rr = ti.qt * kRows + c, tr = rr / ti.group, hr = ti.h * ti.group + rr % ti.group;
-    __hip_bfloat16 *dst =
-        reinterpret_cast<__hip_bfloat16 *>(a.out) + ((int64_t)ti.b * a.width + tr) * a.out_stride + (int64_t)hr * kD;
-#pragma unroll
-    for (int i = 0; i < 16; ++i) dst[16 * g + i] = from_f32<__hip_bfloat16>(NAN);
-  }
-  // the workgroup's key range: up to its first wave's tile's row metadata
-  // and the last live tile's last query
-  TileInfo t0;
-  if (!tile_info_at(a, bh * a.n_qtiles + qb * kPrefillTiles, t0, /*any_split=*/true)) return;  // no live tile
-  // (tiles whose keys would pass max_kv_len took the NaN branch above)
-  const int last_qt = min(qb * kPrefillTiles + kPrefillTiles - 1, (t0.nrows - 1) / kRows);
-  const int t_last = min(min(last_qt * kRows + kRows - 1, t0.nrows - 1) / t0.group,
-                         a.max_kv - 1 - t0.past);
-  const int wg_kv = t0.past + t_last + 1;
-  const int bs = (MODE == 1) ? 16 : a.bs;
-  const int Hkv = a.Hkv;
-  const int32_t *trow = a.tables + (int64_t)t0.row * a.table_stride;
-  const int last_blk = (wg_kv - 1) / bs;
-  const u16 *kp = reinterpret_cast<const u16 *>(a.k);
-  const u16 *vp = reinterpret_cast<const u16 *>(a.v);
-  const int64_t tile_elems = (int64_t)bs * kD;
-
-  // staging: thread tid takes 16-byte units tid + 512 i of the stage's
-  // 2048 (units 0..1023: K, 8 groups x 16 tokens x 8; 1024..2047: V, 8
-  // groups x 64 dims x 2): groups tid / 128 and tid / 128 + 4, the same for
-  // a whole wave, so their block ids are scalar loads (counted apart from
-  // the vector loads: waiting for an id never waits for staged data)
-  u32x4 stg_a[kPUnits], stg_b[kPUnits];
-  const int grp_lo = __builtin_amdgcn_readfirstlane(tid >> 7);
-  // the table is not written while the kernel runs: read through the
-  // constant address space, so a uniform index becomes a scalar load
+  constexpr int T = kPThreads, NU = kPUnits, NB = NU / 2;  // NB: 16-token groups a thread stages
+  __shared__ __align__(16) u16 s_k[2][kPElems];  // [key][dim], 16-byte pieces permuted by key / 2
+  __shared__ __align__(16) u16 s_v[2][kPElems];  // [16-key group][dim][16 keys]
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int q = lane & 31, h = lane >> 5;
+  const int Hkv = a.Hkv, group = a.H / Hkv, bhs = a.batch * Hkv;
+  const int nqb = (a.width * group + kPBlock - 1) / kPBlock;
+  const int qb = nqb - 1 - (int)blockIdx.x / bhs, bh = (int)blockIdx.x % bhs;
+  const int b = bh / Hkv, kvh = bh % Hkv;
   typedef const __attribute__((address_space(4))) int32_t const_i32;
-  const_i32 *trow_c = (const_i32 *)trow;
-  auto blocks_of_stage = [&](int c0, int (&bid)[2]) {
+  const_i32 *meta = (const_i32 *)a.meta;
+  const int trow_i = meta[b], past = meta[a.batch + b], nrows = meta[2 * a.batch + b] * group;
+  const int r0 = qb * kPBlock;
+  if (r0 >= nrows) return;
+  const int bs = (MODE == 1) ? 16 : a.bs;
+  // no key past the call's max_kv_len is read; the rows that would need one
+  // get NaN, by 16-row tiles as in the other kernels
+  const int wg_kv = min(past + (min(r0 + kPBlock, nrows) - 1) / group + 1, a.max_kv);
+  const int wr0 = r0 + kPRows * wave;
+  const int wave_kv = wr0 < nrows ? min(past + min(wr0 + kPRows - 1, nrows - 1) / group + 1, a.max_kv) : 0;
+  const int wave_first = past + wr0 / group;  // position of the wave's first query
+  const int r = min(wr0 + q, nrows - 1), t = r / group, hq = kvh * group + r % group;
+  const bool row_ok = wr0 + q < nrows;
+  const bool overflow = past + min(r / kRows * kRows + kRows - 1, nrows - 1) / group + 1 > a.max_kv;
+  const int qpos = min(past + t, a.max_kv - 1);  // (the bound holds for every row but those)
+
+  // ---- staging: unit tid + T i is 16 bytes of K (i < NB: 4 groups x 16
+  // tokens x 8 pieces) or of V (4 groups x 64 dims x 2); a wave's units of
+  // one i lie in one group, so its block id is a scalar load
+  const u16 *kp = reinterpret_cast<const u16 *>(a.k), *vp = reinterpret_cast<const u16 *>(a.v);
+  const int64_t tile_elems = (int64_t)bs * kD;
+  const int last_blk = (wg_kv - 1) / bs;
+  const_i32 *trow = (const_i32 *)(a.tables + (int64_t)trow_i * a.table_stride);
+  auto group_of = [&](int i) { return (wave * kWave + T * i) >> 7; };
+  auto blocks_of = [&](int c0, int (&bid)[NB]) {
 #pragma unroll
-    for (int h = 0; h < 2; ++h)
-      bid[h] = trow_c[__builtin_amdgcn_readfirstlane(min((c0 + 16 * (grp_lo + 4 * h)) / bs, last_blk))];
+    for (int i = 0; i < NB; ++i)
+      bid[i] = trow[__builtin_amdgcn_readfirstlane(min((c0 + 16 * group_of(i)) / bs, last_blk))];
   };
-  auto unit_of = [&](int i, int &isv, int &grp, int &x) {
-    const int u = tid + i * kPrefillThreads;
-    isv = u >> 10;
-    const int w = u & 1023;
-    grp = w >> 7;
-    x = w & 127;
-  };
-  // Loads are unconditional (a group past the workgroup's keys reads its
-  // clamped block, which is the row's own), so the compiler counts them in
-  // straight-line code and a store waits only for its own stage's loads;
-  // such groups are zeroed when stored.
-  auto stage_load = [&](u32x4 (&stg)[kPUnits], int c0, const int (&bid)[2]) {
+  const int x0 = tid & 127;
+  const int k_off = (x0 >> 3) * kD + (x0 & 7) * 8;        // token x0 / 8, piece x0 % 8
+  const int v_dim = x0 >> 1, v_off = v_dim * bs + (x0 & 1) * 8;  // dim x0 / 2, tokens 8 (x0 % 2) ..
+  // loads are unconditional (a group past the keys reads its clamped block,
+  // which is the row's own) and such groups are zeroed when stored
+  auto stage_load = [&](u32x4 (&stg)[NU], int c0, const int (&bid)[NB]) {
 #pragma unroll
-    for (int i = 0; i < kPUnits; ++i) {
-      int isv, grp, x;
-      unit_of(i, isv, grp, x);
-      const int tok0 = c0 + 16 * grp;
-      const int64_t tile = ((int64_t)bid[grp >> 2] * Hkv + t0.h) * tile_elems;
-      if (!isv) {  // K: token x / 8, dims 8 (x % 8) ..
-        const int tk = x >> 3, dd = (x & 7) * 8;
-        stg[i] = *reinterpret_cast<const u32x4 *>(kp + tile + (int64_t)(tok0 % bs + tk) * kD + dd);
-      } else {  // V: dim x / 2, tokens 8 (x % 2) .. of the group
-        const int dim = x >> 1, t8 = (x & 1) * 8;
-        stg[i] = *reinterpret_cast<const u32x4 *>(vp + tile + (int64_t)dim * bs + tok0 % bs + t8);
-      }
+    for (int i = 0; i < NB; ++i) {
+      const int64_t tile = ((int64_t)bid[i] * Hkv + kvh) * tile_elems;
+      const int in = (c0 + 16 * group_of(i)) % bs;
+      stg[i] = *reinterpret_cast<const u32x4 *>(kp + tile + in * kD + k_off);
+      stg[NB + i] = *reinterpret_cast<const u32x4 *>(vp + tile + in + v_off);
     }
   };
-  auto stage_store = [&](const u32x4 (&stg)[kPUnits], int buf, int c0) {
+  auto stage_store = [&](const u32x4 (&stg)[NU], int buf, int c0) {
 #pragma unroll
-    for (int i = 0; i < kPUnits; ++i) {
-      int isv, grp, x;
-      unit_of(i, isv, grp, x);
-      const u32x4 v = c0 + 16 * grp < wg_kv ? stg[i] : u32x4{0u, 0u, 0u, 0u};
-      if (!isv) {
-        const int tk = x >> 3, dd = (x & 7) * 8;
-        *reinterpret_cast<u32x4 *>(&s_k[buf][(16 * grp + tk) * kPKStride + dd]) = v;
-      } else {
-        const int dim = x >> 1, t8 = (x & 1) * 8;
-        *reinterpret_cast<u32x4 *>(&s_v[buf][(grp * kD + dim) * kPVStride + t8]) = v;
-      }
+    for (int i = 0; i < NB; ++i) {
+      const int grp = group_of(i);
+      const bool live = c0 + 16 * grp < wg_kv;
+      const int key = 16 * grp + (x0 >> 3);
+      const u32x4 zero = u32x4{0u, 0u, 0u, 0u};
+      *reinterpret_cast<u32x4 *>(&s_k[buf][key * kD + (((x0 & 7) ^ ((key >> 1) & 7)) * 8)]) = live ? stg[i] : zero;
+      *reinterpret_cast<u32x4 *>(&s_v[buf][grp * (16 * kD) + x0 * 8]) = live ? stg[NB + i] : zero;
     }
   };
 
-  // this wave's queries
-  const int r = live ? ti.qt * kRows + c : 0;
-  const bool row_ok = live && r < ti.nrows;
-  const int t = row_ok ? r / ti.group : 0;
-  const int hq = live ? ti.h * ti.group + (row_ok ? r % ti.group : 0) : 0;
-  const int qpos = t0.past + t;
-  const int my_kv = live ? ti.kv_len : 0;
-  const float c2 = a.scale * 1.4426950408889634f;  // scores in log2 units
-  bf16x8 qop[2];
+  // ---- this wave's queries: step s holds dims 16 s + 8 h ..
+  bf16x8 qop[4];
   {
-    u32x4 raw[2] = {{0u, 0u, 0u, 0u}, {0u, 0u, 0u, 0u}};
-    if (row_ok) {
-      const u16 *qrow =
-          reinterpret_cast<const u16 *>(a.q) + ((int64_t)t0.b * a.width + t) * a.q_stride + (int64_t)hq * kD;
-      raw[0] = *reinterpret_cast<const u32x4 *>(qrow + 8 * g);
-      raw[1] = *reinterpret_cast<const u32x4 *>(qrow + 32 + 8 * g);
-    }
-    qop[0] = __builtin_bit_cast(bf16x8, raw[0]);
-    qop[1] = __builtin_bit_cast(bf16x8, raw[1]);
+    const u16 *qrow = reinterpret_cast<const u16 *>(a.q) + ((int64_t)b * a.width + t) * a.q_stride + (int64_t)hq * kD;
+#pragma unroll
+    for (int s = 0; s < 4; ++s)
+      qop[s] = __builtin_bit_cast(bf16x8, *reinterpret_cast<const u32x4 *>(qrow + 16 * s + 8 * h));
   }
-  if (a.rope && row_ok) {
-    const float *cs = a.cos_t + (int64_t)qpos * (kD / 2) + 8 * g;
-    const float *sn = a.sin_t + (int64_t)qpos * (kD / 2) + 8 * g;
+  if (a.rope) {
 #pragma unroll
-    for (int j = 0; j < 8; ++j) {
-      float y1, y2;
-      rope_pair((float)qop[0][j], (float)qop[1][j], cs[j], sn[j], y1, y2);
-      qop[0][j] = (__bf16)y1;
-      qop[1][j] = (__bf16)y2;
-    }
-  }
-  f32x4 o[4];
+    for (int s = 0; s < 2; ++s) {
+      const float *cs = a.cos_t + (int64_t)qpos * (kD / 2) + 16 * s + 8 * h;
+      const float *sn = a.sin_t + (int64_t)qpos * (kD / 2) + 16 * s + 8 * h;
 #pragma unroll
-  for (int tt = 0; tt < 4; ++tt) o[tt] = f32x4{0.f, 0.f, 0.f, 0.f};
-  float m = -INFINITY, l = 0.0f;
-  // one 64-token step (half hs of the stage) from LDS buffer buf
-  auto compute = [&](int c0, int buf, int hs) {
-    float sv[16];
-#pragma unroll
-    for (int ch = 0; ch < 2; ++ch) {
-#pragma unroll
-      for (int hf = 0; hf < 2; ++hf) {
-        const int tk = 64 * hs + 32 * ch + 8 * (c >> 2) + 4 * hf + (c & 3);  // token within the stage
-        const u16 *kr = &s_k[buf][tk * kPKStride + 8 * g];
-        const u32x4 k0 = *reinterpret_cast<const u32x4 *>(kr);
-        const u32x4 k1 = *reinterpret_cast<const u32x4 *>(kr + 32);
-        f32x4 sc = f32x4{0.f, 0.f, 0.f, 0.f};
-        sc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, k0), qop[0], sc, 0, 0, 0);
-        sc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, k1), qop[1], sc, 0, 0, 0);
-#pragma unroll
-        for (int i = 0; i < 4; ++i) sv[8 * ch + 4 * hf + i] = sc[i] * c2;
+      for (int j = 0; j < 8; ++j) {
+        float y1, y2;
+        rope_pair((float)qop[s][j], (float)qop[s + 2][j], cs[j], sn[j], y1, y2);
+        qop[s][j] = (__bf16)y1;
+        qop[s + 2][j] = (__bf16)y2;
       }
     }
-    if (c0 + 64 > t0.past) {
+  }
+  // scores in log2 units are c2 s; the softmax takes the maximum of s, which
+  // needs c2 > 0: a negative scale changes q's sign instead (a zero one is the
+  // smallest normal number, whose products vanish against a maximum)
+  float c2 = a.scale * 1.4426950408889634f;
+  if (c2 < 0.0f) {
+    c2 = -c2;
 #pragma unroll
-      for (int ch = 0; ch < 2; ++ch)
+    for (int s = 0; s < 4; ++s) qop[s] = __builtin_bit_cast(bf16x8, __builtin_bit_cast(u32x4, qop[s]) ^ 0x80008000u);
+  }
+  if (c2 == 0.0f) c2 = 1.17549435e-38f;
+
+  f32x16 o[2];
 #pragma unroll
-        for (int j = 0; j < 8; ++j) {
-          const int pos = c0 + 32 * ch + 8 * g + j;
-          if (!(row_ok && pos <= qpos && pos < my_kv)) sv[8 * ch + j] = -INFINITY;
+  for (int i = 0; i < 16; ++i) o[0][i] = o[1][i] = 0.0f;
+  float m = -INFINITY, l = 0.0f;  // m: the row's maximum of c2 s; l: this half-wave's part of the sum
+  const int key_row = 16 * (q >> 4) + 8 * ((q >> 2) & 1) + 4 * ((q >> 3) & 1) + (q & 3);
+  auto compute = [&](int c0, int buf) {
+    f32x16 sc[2];
+#pragma unroll
+    for (int kt = 0; kt < 2; ++kt) {
+      const int key = 32 * kt + key_row;
+      f32x16 d;
+#pragma unroll
+      for (int i = 0; i < 16; ++i) d[i] = 0.0f;
+#pragma unroll
+      for (int s = 0; s < 4; ++s) {
+        const u32x4 kv = *reinterpret_cast<const u32x4 *>(&s_k[buf][key * kD + (((2 * s + h) ^ ((key >> 1) & 7)) * 8)]);
+        d = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, kv), qop[s], d, 0, 0, 0);
+      }
+      sc[kt] = d;
+    }
+    if (c0 + kPStage - 1 > wave_first) {  // some key lies past some query
+#pragma unroll
+      for (int kt = 0; kt < 2; ++kt)
+#pragma unroll
+        for (int i = 0; i < 16; ++i) {
+          const int pos = c0 + 32 * kt + 16 * (i >> 3) + 8 * h + (i & 7);
+          if (pos > qpos) sc[kt][i] = -INFINITY;
         }
     }
-    online_update<16>(sv, m, l, o);
+    float mx = sc[0][0];
 #pragma unroll
-    for (int ch = 0; ch < 2; ++ch) {
-      bf16x8 pop;
+    for (int kt = 0; kt < 2; ++kt)
 #pragma unroll
-      for (int j = 0; j < 8; ++j) pop[j] = (__bf16)sv[8 * ch + j];
-      // lane group g's 8 tokens: 16-token group 2 ch + g / 2, tokens 8 (g % 2) ..
-      const u16 *vr = &s_v[buf][((4 * hs + 2 * ch + (g >> 1)) * kD + c) * kPVStride + 8 * (g & 1)];
+      for (int i = 0; i < 16; ++i) mx = fmaxf(mx, sc[kt][i]);
+    mx = fmaxf(mx, other_half(mx));
+    // m, the base of the exponents, moves only when a row's maximum has left
+    // it by more than 8 (p up to 256, exact in the same way: a step that moves
+    // it rescales 32 values of O, which nearly every step did)
+    const float m_new = fmaxf(m, mx * c2);
+    if (__builtin_amdgcn_ballot_w64(m_new > m + 8.0f)) {
+      // (exp2(-inf) = 0 where nothing was seen before; a row with no finite
+      // score yet keeps 0 as the base, so that -inf - -inf never arises)
+      const float f = __builtin_amdgcn_exp2f(m - (m_new == -INFINITY ? 0.0f : m_new));
+      l *= f;
 #pragma unroll
-      for (int tt = 0; tt < 4; ++tt) {
-        const u32x4 vv = *reinterpret_cast<const u32x4 *>(vr + 16 * tt * kPVStride);
-        o[tt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, vv), pop, o[tt], 0, 0, 0);
+      for (int tt = 0; tt < 2; ++tt)
+#pragma unroll
+        for (int i = 0; i < 16; ++i) o[tt][i] *= f;
+      m = m_new;
+    }
+    const float base = m == -INFINITY ? 0.0f : m;
+    bf16x8 pop[2][2];
+#pragma unroll
+    for (int kt = 0; kt < 2; ++kt)
+#pragma unroll
+      for (int i = 0; i < 16; ++i) {
+        const float p = __builtin_amdgcn_exp2f(__builtin_fmaf(sc[kt][i], c2, -base));
+        l += p;
+        pop[kt][i >> 3][i & 7] = (__bf16)p;
+      }
+#pragma unroll
+    for (int kt = 0; kt < 2; ++kt)
+#pragma unroll
+      for (int u = 0; u < 2; ++u)
+#pragma unroll
+        for (int tt = 0; tt < 2; ++tt) {
+          const u32x4 vv =
+              *reinterpret_cast<const u32x4 *>(&s_v[buf][((2 * kt + u) * kD + 32 * tt + q) * 16 + 8 * h]);
+          o[tt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, vv), pop[kt][u], o[tt], 0, 0, 0);
+        }
+  };
+  // stage s lives in LDS buffer s % 2; its loads go out during stage s - 1
+  u32x4 stg[NU];
+  int bid[NB];
+  blocks_of(0, bid);
+  stage_load(stg, 0, bid);
+  blocks_of(kPStage, bid);
+  stage_store(stg, 0, 0);
+  __syncthreads();
+  for (int c0 = 0, buf = 0; c0 < wg_kv; c0 += kPStage, buf ^= 1) {
+    stage_load(stg, c0 + kPStage, bid);
+    blocks_of(c0 + 2 * kPStage, bid);
+    if (c0 < wave_kv) compute(c0, buf);
+    stage_store(stg, buf ^ 1, c0 + kPStage);
+    __syncthreads();
+  }
+  if (!row_ok) return;
+  l += other_half(l);
+  // lane (q, h) holds dims 32 tt + 8 (i / 4) + 4 h + i % 4 of its query
+  const float inv = overflow ? NAN : 1.0f / l;
+  u16 *dst = reinterpret_cast<u16 *>(a.out) + ((int64_t)b * a.width + t) * a.out_stride + (int64_t)hq * kD + 4 * h;
+  const bool aligned = (((uintptr_t)a.out | (uintptr_t)(a.out_stride * 2)) & 7) == 0;
+#pragma unroll
+  for (int tt = 0; tt < 2; ++tt)
+#pragma unroll
+    for (int i4 = 0; i4 < 4; ++i4) {
+      u16 v[4];
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+        v[i] = __builtin_bit_cast(u16, from_f32<__hip_bfloat16>(o[tt][4 * i4 + i] * inv));
+      u16 *dd = dst + 32 * tt + 8 * i4;
+      if (aligned) {
+        *reinterpret_cast<u32x2 *>(dd) =
+            u32x2{(uint32_t)v[0] | ((uint32_t)v[1] << 16), (uint32_t)v[2] | ((uint32_t)v[3] << 16)};
+      } else {
+#pragma unroll
+        for (int i = 0; i < 4; ++i) dd[i] = v[i];
       }
     }
-  };
-  // stage s lives in LDS buffer s % 3; its loads go out during stage s - 2
-  int bid[2];
-  blocks_of_stage(0, bid);
-  stage_load(stg_a, 0, bid);
-  blocks_of_stage(kPStage, bid);
-  stage_store(stg_a, 0, 0);
-  stage_load(stg_a, kPStage, bid);  // stage 1, stored during stage 0
-  blocks_of_stage(2 * kPStage, bid);
-  __syncthreads();
-  auto stage_step = [&](int c0, int buf, u32x4 (&held)[kPUnits], u32x4 (&ahead)[kPUnits]) {
-    // held: stage c0 + kPStage's data, stored now; ahead: stage c0 + 2 kPStage's, loaded now
-    // (every step loads and stores, also past the keys: no branch around a
-    // load, so each wait is for exactly the loads it needs)
-    stage_load(ahead, c0 + 2 * kPStage, bid);
-    blocks_of_stage(c0 + 3 * kPStage, bid);
-    if (c0 < my_kv) compute(c0, buf, 0);
-    if (c0 + 64 < my_kv) compute(c0 + 64, buf, 1);
-    stage_store(held, buf == 2 ? 0 : buf + 1, c0 + kPStage);
-    __syncthreads();
-  };
-  int buf = 0;
-  for (int c0 = 0; c0 < wg_kv; c0 += 2 * kPStage) {
-    stage_step(c0, buf, stg_a, stg_b);
-    buf = buf == 2 ? 0 : buf + 1;
-    if (c0 + kPStage >= wg_kv) break;
-    stage_step(c0 + kPStage, buf, stg_b, stg_a);
-    buf = buf == 2 ? 0 : buf + 1;
-  }
-  // O^T accumulators: lane (c, g) holds dims 16 tt + 4 g + i of query row c
-  if (row_ok) {
-    __hip_bfloat16 *dst = reinterpret_cast<__hip_bfloat16 *>(a.out) + ((int64_t)t0.b * a.width + t) * a.out_stride +
-                          (int64_t)hq * kD;
-#pragma unroll
-    for (int tt = 0; tt < 4; ++tt)
-#pragma unroll
-      for (int i = 0; i < 4; ++i) dst[16 * tt + 4 * g + i] = from_f32<__hip_bfloat16>(o[tt][i] / l);
-  }
 }
 
 // ---------------------------------------------------------------- fp32 ----
@@ -1845,11 +1856,11 @@ static int run_attention(AttnArgs &a, const AttnPlan &plan, int dtype, int32_t b
                                 const_cast<void *>(a.k), const_cast<void *>(a.v), /*kv_only=*/true, s);
       if (st != SPECDEC_OK) return st;
     }
-    const int64_t blocks = (int64_t)a.batch * a.Hkv * ((a.n_qtiles + kPrefillTiles - 1) / kPrefillTiles);
-    if (blocks > INT32_MAX) return SPECDEC_EUNSUPPORTED;
-    dim3 pgrid((unsigned)blocks), pblock(kPrefillThreads);
-    if (block_size == 16) attention_prefill_kernel<1><<<pgrid, pblock, 0, s>>>(a);
-    else attention_prefill_kernel<2><<<pgrid, pblock, 0, s>>>(a);
+    const int64_t heads = (int64_t)a.batch * a.Hkv, rows = (int64_t)a.width * (a.H / a.Hkv);
+    const int64_t blocks = heads * ((rows + kPBlock - 1) / kPBlock);
+    if (blocks > INT32_MAX || rows > INT32_MAX - kPBlock) return SPECDEC_EUNSUPPORTED;
+    if (block_size == 16) attention_prefill_kernel<1><<<(unsigned)blocks, kPThreads, 0, s>>>(a);
+    else attention_prefill_kernel<2><<<(unsigned)blocks, kPThreads, 0, s>>>(a);
     return launch_status();
   }
   if (plan.decode) {

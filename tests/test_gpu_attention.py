@@ -823,3 +823,49 @@ def test_short_token_buffers_are_refused_before_launch():
     # the same buffers at full length run
     ops.paged_attention(q, q.stride(1), *args, out, out.stride(1))
     torch.cuda.synchronize()
+
+
+# widths at the edges of the prompt kernel's 32-row waves, 128-row workgroups
+# and 64-key stages, with query heads that end a wave inside a token
+@pytest.mark.parametrize("t_new,lengths,heads,bs", [(17, [1, 63], (8, 8), 16), (32, [64, 31], (4, 4), 32),
+                                                    (33, [1, 200], (9, 3), 16), (43, [85, 20], (9, 3), 48),
+                                                    (128, [1, 64], (4, 4), 16), (129, [300, 3], (4, 2), 16),
+                                                    (20, [700, 45], (16, 1), 16)])
+def test_prefill_edges_match_oracle(t_new, lengths, heads, bs):
+    for got, want in run_case(2, lengths, *heads, bs, torch.bfloat16, t_new, seed=t_new):
+        err = (got - want).abs()
+        # bf16 outputs of magnitude up to 2 (a step of 2^-7), p rounded to bf16
+        assert err.max().item() < 2e-2 and err.mean().item() < 2e-3, (err.max().item(), err.mean().item())
+
+
+def test_prefill_rows_do_not_depend_on_the_batch_and_scales_of_any_sign():
+    d, h, hkv, bs = 64, 6, 2, 16
+    g = torch.Generator().manual_seed(3)
+    lengths, t_new = [5, 140, 64], [90, 33, 71]
+    cache = make_cache(1, hkv, d, 80, bs, torch.bfloat16, 2)
+    for s in range(3):
+        cache.add(s)
+    k, v = (torch.randn(3, hkv, 240, d, generator=g).to(torch.bfloat16) for _ in range(2))
+    total = [m + n for m, n in zip(lengths, t_new)]
+    step = cache.append([0, 1, 2], total)
+    cache.write(0, step, k[:, :, :max(total)].cuda(), v[:, :, :max(total)].cuda())
+    q = torch.randn(3, 90, h * d, generator=g).to(torch.bfloat16).cuda()
+    rows = step.meta[0].tolist()
+
+    def call(which, scale):
+        meta = torch.tensor([[rows[i] for i in which], [lengths[i] for i in which], [t_new[i] for i in which]],
+                            dtype=torch.int32, device="cuda")
+        out = torch.zeros(len(which), 90, h * d, dtype=torch.bfloat16, device="cuda")
+        x = q[which].contiguous()
+        ops.paged_attention(x, x.stride(1), cache.k[0], cache.v[0], cache.table_tensor, meta, len(which), 90, h, hkv,
+                            d, bs, scale, max(total), out, out.stride(1))
+        return out
+
+    for scale in (0.125, -0.2, 0.0):
+        together = call([0, 1, 2], scale)
+        want = of.attention(q.view(3, 90, h, d).transpose(1, 2).float().cpu(), k.float()[:, :, :max(total)],
+                            v.float()[:, :, :max(total)], torch.tensor(lengths), torch.tensor(total), scale)
+        got = together.view(3, 90, h, d).transpose(1, 2).float().cpu()
+        for b in range(3):
+            assert torch.equal(call([b], scale), together[b:b + 1]), (scale, b)
+            assert (got[b, :, :t_new[b]] - want[b, :, :t_new[b]]).abs().max().item() < 2e-2, (scale, b)
