@@ -473,6 +473,25 @@ int specdec_head_probabilities(const void *x, int64_t x_stride, const void *w, i
                                void *workspace, int64_t workspace_bytes, int32_t spin,
                                void *stream);
 
+/* Floats of the workspace of specdec_head_softmax for `rows` rows of `vocab`
+ * (needs no initialisation). */
+int specdec_head_softmax_workspace(int64_t rows, int64_t vocab, int64_t *floats);
+
+/* The output head and probabilities for any number of rows (at most 65535):
+ * out [rows, vocab] fp32 (out_stride apart) = one-hot of each row's argmax
+ * (lowest id among ties) at temperature 0, else softmax(logits /
+ * temperature), with the logits of specdec_head_logits; index_out as in
+ * specdec_head_probabilities.  Two launches: the logits go to `out` with
+ * statistics per slice of the vocab to `workspace`, then each row is
+ * finished in place over many workgroups.  Nothing is exchanged within a
+ * launch.  Calls that share a workspace must be ordered on one stream.
+ * Replaces lm/forward.py:71-84 followed by lm/sampling.py:13-18. */
+int specdec_head_softmax(const void *x, int64_t x_stride, const void *w, int64_t w_stride,
+                         int64_t rows, int64_t hidden, int64_t vocab, float temperature,
+                         float *out, int64_t out_stride, int64_t *index_out,
+                         int64_t index_stride, float *workspace, int64_t workspace_floats,
+                         void *stream);
+
 /* fp32 split partials the library holds per GPU for
  * specdec_paged_attention_static (8 MiB). */
 #define SPECDEC_STATIC_PARTIAL_FLOATS (2 * 1024 * 1024)

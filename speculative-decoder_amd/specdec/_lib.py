@@ -48,6 +48,8 @@ SIGNATURES: dict[str, list] = {
     "specdec_linear": [P, I64, P, I64, I32, I64, I64, I64, P, I64, I32, P],
     "specdec_linear_silu": [P, I64, P, I64, I32, I64, I64, I64, P, I64, I64, c_float, P, I64, P],
     "specdec_head_probabilities": [P, I64, P, I64, I64, I64, I64, c_float, P, I64, P, I64, P, I64, P, I64, I32, P],
+    "specdec_head_softmax_workspace": [I64, I64, P],
+    "specdec_head_softmax": [P, I64, P, I64, I64, I64, I64, c_float, P, I64, P, I64, P, I64, P],
     "specdec_paged_attention_static": [P, c_int, I64, P, P, P, I64, P, I32, I32, I32, I32, I32, I32, c_float,
                                        I32, I32, P, I64, P],
 }

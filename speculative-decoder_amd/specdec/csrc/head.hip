@@ -58,6 +58,9 @@ constexpr int kHMaxTpw = 16;                // tiles (and waves) per workgroup
 constexpr int kHSlice = kHMaxTpw * kHT;     // vocab rows per workgroup, at most
 constexpr int kHXPad = 8;                   // bf16 padding per staged hidden row (LDS banks)
 constexpr int kHXElems = kHT * (2048 + kHXPad);  // staged hidden elements (bf16)
+// staged hidden elements of a head_logits pass of more than 16 rows (132 KB of
+// the 160): at 64 rows the 2048-wide head's k-steps are two chunks
+constexpr int kHXWide = 4 * kHT * (1024 + kHXPad);
 constexpr int kHMaxGrid = 256;              // workgroups of a fused call, at most
 constexpr int kHFusedRows = 16;             // hidden rows of a fused call, at most
 // workspace words: two arrival counters, the call epoch, then kHCopies
@@ -98,33 +101,47 @@ struct HeadArgs {
 };
 
 // ---- the logits of one vocab tile --------------------------------------
-// Stage hidden rows r0 .. r0 + 16*NCT - 1 (zeros past M), k-steps
-// [k0, k0 + kn), into s_x with row stride xs elements; the steps up to the
-// next multiple of KB are staged as zeros.  A thread's loads of a round go
-// out together, then its LDS stores.
-template <int NCT, int KB>
-__device__ __forceinline__ void stage_x(const HeadArgs &a, uint16_t *s_x, int xs, int r0, int k0, int kn) {
-  constexpr int kU = 8;  // 16-byte units per thread per round
+// Hidden rows r0 .. r0 + 16*NCT - 1 (zeros past M), k-steps [k0, k0 + kn), as
+// 16-byte units of s_x with row stride xs elements; the steps up to the next
+// multiple of KB are zeros.  stage_load takes kU units a thread from unit u0
+// on into registers (all loads go out together), stage_store puts them into
+// LDS.
+constexpr int kHStageUnits = 12;
+struct XStage {
+  int k0, kn, per_row, total;
+};
+template <int NCT, int KB> __device__ __forceinline__ XStage stage_of(int k0, int kn) {
   const int per_row = (kn + KB - 1) / KB * KB * 4;
-  const int valid = kn * 4;
-  const int total = kHT * NCT * per_row;
-  for (int u0 = 0; u0 < total; u0 += kU * (int)blockDim.x) {
+  return XStage{k0, kn, per_row, kHT * NCT * per_row};
+}
+template <int U>
+__device__ __forceinline__ void stage_load(const HeadArgs &a, const XStage &st, int r0, int u0, u32x4 (&v)[U]) {
+#pragma unroll
+  for (int i = 0; i < U; ++i) {
+    const int u = u0 + i * (int)blockDim.x + (int)threadIdx.x;
+    const int r = u / st.per_row, j = u - r * st.per_row;
+    v[i] = u32x4{0u, 0u, 0u, 0u};
+    if (u < st.total && r0 + r < a.M && j < st.kn * 4)
+      v[i] = *reinterpret_cast<const u32x4 *>(a.x + (int64_t)(r0 + r) * a.x_stride + (int64_t)st.k0 * 32 + 8 * j);
+  }
+}
+template <int U>
+__device__ __forceinline__ void stage_store(const XStage &st, uint16_t *s_x, int xs, int u0, const u32x4 (&v)[U]) {
+#pragma unroll
+  for (int i = 0; i < U; ++i) {
+    const int u = u0 + i * (int)blockDim.x + (int)threadIdx.x;
+    const int r = u / st.per_row, j = u - r * st.per_row;
+    if (u < st.total) *reinterpret_cast<u32x4 *>(s_x + r * xs + 8 * j) = v[i];
+  }
+}
+// The units from u0 on, a round at a time.
+__device__ __forceinline__ void stage_rest(const HeadArgs &a, const XStage &st, uint16_t *s_x, int xs, int r0, int u0) {
+  constexpr int kU = 8;
+  for (; u0 < st.total; u0 += kU * (int)blockDim.x) {
     u32x4 v[kU];
-#pragma unroll
-    for (int i = 0; i < kU; ++i) {
-      const int u = u0 + i * (int)blockDim.x + (int)threadIdx.x;
-      const int r = u / per_row, j = u - r * per_row;
-      v[i] = u32x4{0u, 0u, 0u, 0u};
-      if (u < total && r0 + r < a.M && j < valid)
-        v[i] = *reinterpret_cast<const u32x4 *>(a.x + (int64_t)(r0 + r) * a.x_stride + (int64_t)k0 * 32 + 8 * j);
-    }
+    stage_load<kU>(a, st, r0, u0, v);
     __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-    for (int i = 0; i < kU; ++i) {
-      const int u = u0 + i * (int)blockDim.x + (int)threadIdx.x;
-      const int r = u / per_row, j = u - r * per_row;
-      if (u < total) *reinterpret_cast<u32x4 *>(s_x + r * xs + 8 * j) = v[i];
-    }
+    stage_store<kU>(st, s_x, xs, u0, v);
   }
 }
 
@@ -134,13 +151,15 @@ __device__ __forceinline__ void stage_x(const HeadArgs &a, uint16_t *s_x, int xs
 // thread of the workgroup calls it).
 // Per chunk the W rows stream in batches of KB k-steps, the next batch's
 // loads in flight while one is multiplied; the chunk's first batch is
-// issued before its hidden rows are staged.  The loop body issues its loads
+// issued before its hidden rows are staged, and (AHEAD) most of the next
+// chunk's hidden rows are loaded into registers while one is multiplied, so
+// that the chunk's end costs two barriers and LDS writes, not a round trip.  The loop body issues its loads
 // without conditions (the last one or two batches are peeled), so the
 // compiler's wait counts stay exact; the steps of a partial last batch
 // re-read step kn - 1 and meet staged zeros, adding exact zeros.  The
 // scheduling barriers keep each batch's loads ahead of the previous batch's
 // multiplies, where the compiler would otherwise sink them.
-template <int NCT, int KB>
+template <int NCT, int KB, bool AHEAD = false>
 __device__ __forceinline__ void slice_logits(const HeadArgs &a, uint16_t *s_x, int j, int r0, f32x4 (&acc)[NCT]) {
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, c = lane & 15, g = lane >> 4;
   const int tile = j * a.tpw + wave;
@@ -173,14 +192,25 @@ __device__ __forceinline__ void slice_logits(const HeadArgs &a, uint16_t *s_x, i
       }
     }
   };
+  constexpr int kAhead = AHEAD ? kHStageUnits : 1;
+  u32x4 xv[kAhead];
   for (int k0 = 0; k0 < a.steps; k0 += a.kc) {
     const int kn = min(a.kc, a.steps - k0);
     const int nb = (kn + KB - 1) / KB;
+    const XStage st = stage_of<NCT, KB>(k0, kn);
     if (mine) issue(A0, k0, kn, 0);
     __builtin_amdgcn_sched_barrier(0);
     if (k0 > 0) __syncthreads();
-    stage_x<NCT, KB>(a, s_x, xs, r0, k0, kn);
+    if (AHEAD && k0 > 0) {
+      stage_store<kAhead>(st, s_x, xs, 0, xv);
+      stage_rest(a, st, s_x, xs, r0, kAhead * (int)blockDim.x);
+    } else {
+      stage_rest(a, st, s_x, xs, r0, 0);
+    }
     __syncthreads();
+    if (AHEAD && k0 + a.kc < a.steps)
+      stage_load<kAhead>(a, stage_of<NCT, KB>(k0 + a.kc, min(a.kc, a.steps - k0 - a.kc)), r0, 0, xv);
+    __builtin_amdgcn_sched_barrier(0);
     if (mine) {
       int b = 0;
       for (; b + 2 < nb; b += 2) {
@@ -261,20 +291,173 @@ __device__ __forceinline__ void store_logits4(float *row_ptr, int v0, int V, con
 }
 
 // ---- kernels --------------------------------------------------------------
-// Logits only: grid (slices, passes of 16*NCT hidden rows).
-template <int NCT, int KB>
-__global__ __launch_bounds__(1024) void head_logits_kernel(HeadArgs a) {
-  __shared__ __align__(16) uint16_t s_x[kHXElems];
-  const int r0 = blockIdx.y * kHT * NCT;
+// The logits: slices x passes of 16*NCT hidden rows, at most TH threads (a
+// wave a tile; 768, three waves a SIMD, leave 168 registers).  The passes of
+// a slice are eight workgroups apart, so they run together on one XCD and the
+// slice's W comes from memory once (72 rows of the 2048-wide head, two passes:
+// 84 us with all slices of the first pass first).
+// With `stats` each row's statistics of the slice follow: the maximum y of
+// l / T and the sum of 2^((y' - y) log2 e) (T > 0), or the maximum logit and
+// its lowest index (T = 0), for head_finish_kernel to fold.
+struct HeadStats {
+  float *stats;  // [M, slices, 2], or null
+  int slices;
+};
+template <int NCT, int KB, int TH>
+__global__ __launch_bounds__(TH) void head_logits_kernel(HeadArgs a, HeadStats hs, int passes) {
+  extern __shared__ __align__(16) uint16_t s_x[];
+  __shared__ float s_st[kHMaxTpw][kHT * NCT][2];
+  const int slice = blockIdx.x / (8 * passes) * 8 + blockIdx.x % 8, pass = blockIdx.x / 8 % passes;
+  if (slice >= hs.slices) return;
+  const int r0 = pass * kHT * NCT;
   f32x4 acc[NCT];
-  slice_logits<NCT, KB>(a, s_x, blockIdx.x, r0, acc);
+  slice_logits<NCT, KB, (NCT > 1 && TH <= 768)>(a, s_x, slice, r0, acc);
   const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, c = lane & 15, g = lane >> 4;
-  const int tile = blockIdx.x * a.tpw + wave;
-  if (wave >= a.tpw || tile >= a.tiles) return;
+  const int tile = slice * a.tpw + wave;
+  const bool mine = wave < a.tpw && tile < a.tiles;
+  const int v0 = tile * kHT + 4 * g;
+  if (mine) {
+#pragma unroll
+    for (int ct = 0; ct < NCT; ++ct) {
+      const int r = r0 + ct * kHT + c;
+      if (r < a.M) store_logits4(a.logits + (int64_t)r * a.logits_stride, v0, a.V, acc[ct], a.vec_logits);
+    }
+  }
+  if (!hs.stats) return;
 #pragma unroll
   for (int ct = 0; ct < NCT; ++ct) {
-    const int r = r0 + ct * kHT + c;
-    if (r < a.M) store_logits4(a.logits + (int64_t)r * a.logits_stride, tile * kHT + 4 * g, a.V, acc[ct], a.vec_logits);
+    float m = -INFINITY, x = 0.0f;
+    if (a.temperature == 0.0f) {
+      int best = INT32_MAX;
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+        if (mine && v0 + i < a.V) argmax_keep(m, best, acc[ct][i], v0 + i);
+#pragma unroll
+      for (int off = 16; off < 64; off <<= 1) {
+        const float om = __shfl_xor(m, off, 64);
+        const int ob = __shfl_xor(best, off, 64);
+        argmax_keep(m, best, om, ob);
+      }
+      x = __int_as_float(best);
+    } else {
+      float y[4];
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        y[i] = mine && v0 + i < a.V ? scaled(a, acc[ct][i]) : -INFINITY;
+        m = fmaxf(m, y[i]);
+      }
+      m = fmaxf(m, __shfl_xor(m, 16, 64));
+      m = fmaxf(m, __shfl_xor(m, 32, 64));
+      const float base = m == -INFINITY ? 0.0f : m;
+#pragma unroll
+      for (int i = 0; i < 4; ++i) x += __builtin_amdgcn_exp2f((y[i] - base) * kHLog2e);
+      x += __shfl_xor(x, 16, 64);
+      x += __shfl_xor(x, 32, 64);
+    }
+    if (g == 0) {
+      s_st[wave][ct * kHT + c][0] = m;
+      s_st[wave][ct * kHT + c][1] = x;
+    }
+  }
+  __syncthreads();
+  const int nw = blockDim.x >> 6;
+  for (int r = threadIdx.x; r < kHT * NCT; r += blockDim.x) {
+    if (r0 + r >= a.M) break;
+    float m = s_st[0][r][0], x = s_st[0][r][1];
+    if (a.temperature == 0.0f) {
+      int best = __float_as_int(x);
+      for (int w = 1; w < nw; ++w) argmax_keep(m, best, s_st[w][r][0], __float_as_int(s_st[w][r][1]));
+      x = __int_as_float(best);
+    } else {
+      for (int w = 1; w < nw; ++w) m = fmaxf(m, s_st[w][r][0]);
+      const float base = m == -INFINITY ? 0.0f : m;
+      x = 0.0f;
+      for (int w = 0; w < nw; ++w) x += s_st[w][r][1] * __builtin_amdgcn_exp2f((s_st[w][r][0] - base) * kHLog2e);
+    }
+    float *dst = hs.stats + ((int64_t)(r0 + r) * hs.slices + slice) * 2;
+    dst[0] = m;
+    dst[1] = x;
+  }
+}
+
+// The rows' probabilities from their logits (in place: a thread's elements
+// are read before it writes them) and the slices' statistics: a workgroup
+// folds its row's statistics, in a fixed order, while its kHFinish logits are
+// on their way.  The one-workgroup-per-row softmax kernel leaves most compute
+// units idle: 12.9 us for 40 rows of 49152.
+constexpr int kHFinishThreads = 256, kHFinishVec = 4;
+constexpr int kHFinish = kHFinishThreads * kHFinishVec * 4;  // logits of a workgroup
+__global__ __launch_bounds__(kHFinishThreads) void head_finish_kernel(HeadArgs a, HeadStats hs) {
+  __shared__ float s_m[kHFinishThreads / 64], s_x[kHFinishThreads / 64];
+  const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
+  const int r = blockIdx.y, e0 = blockIdx.x * kHFinish;
+  float *row = a.out + (int64_t)r * a.out_stride;
+  f32x4 v[kHFinishVec];
+#pragma unroll
+  for (int k = 0; k < kHFinishVec; ++k) {
+    const int e = e0 + (k * kHFinishThreads + tid) * 4;
+    v[k] = f32x4{0.f, 0.f, 0.f, 0.f};
+    if (a.vec_out && e + 3 < a.V) v[k] = *reinterpret_cast<const f32x4 *>(row + e);
+    else {
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+        if (e + i < a.V) v[k][i] = row[e + i];
+    }
+  }
+  const float *st = hs.stats + (int64_t)r * hs.slices * 2;
+  const bool hot = a.temperature == 0.0f;
+  float m = -INFINITY, x = 0.0f;
+  int best = INT32_MAX;
+  for (int j = tid; j < hs.slices; j += kHFinishThreads) {
+    const float2 sj = *reinterpret_cast<const float2 *>(st + 2 * j);
+    if (hot) {
+      argmax_keep(m, best, sj.x, __float_as_int(sj.y));
+    } else {
+      const float mn = fmaxf(m, sj.x), base = mn == -INFINITY ? 0.0f : mn;
+      x = x * __builtin_amdgcn_exp2f((m - base) * kHLog2e) + sj.y * __builtin_amdgcn_exp2f((sj.x - base) * kHLog2e);
+      m = mn;
+    }
+  }
+  float mw;
+  if (hot) {
+    mw = m;
+    wave_argmax_dpp(mw, best);
+    x = __int_as_float(best);
+  } else {
+    mw = wave_max_dpp(m);
+    const float base = mw == -INFINITY ? 0.0f : mw;
+    x = wave_sum_dpp(x * __builtin_amdgcn_exp2f((m - base) * kHLog2e));
+  }
+  if (lane == 0) {
+    s_m[wave] = mw;
+    s_x[wave] = x;
+  }
+  __syncthreads();
+  float M = s_m[0];
+  int hot_i = __float_as_int(s_x[0]);
+  float S = 0.0f;
+  if (hot) {
+#pragma unroll
+    for (int w = 1; w < kHFinishThreads / 64; ++w) argmax_keep(M, hot_i, s_m[w], __float_as_int(s_x[w]));
+    hot_i = min(hot_i, a.V - 1);  // a row of NaN alone has no maximum: an id of the vocabulary all the same
+    if (a.index_out && blockIdx.x == 0 && tid == 0) a.index_out[(int64_t)r * a.index_stride] = hot_i;
+  } else {
+#pragma unroll
+    for (int w = 1; w < kHFinishThreads / 64; ++w) M = fmaxf(M, s_m[w]);
+    const float base = M == -INFINITY ? 0.0f : M;
+#pragma unroll
+    for (int w = 0; w < kHFinishThreads / 64; ++w) S += s_x[w] * __builtin_amdgcn_exp2f((s_m[w] - base) * kHLog2e);
+  }
+  const float inv = 1.0f / S;
+#pragma unroll
+  for (int k = 0; k < kHFinishVec; ++k) {
+    const int e = e0 + (k * kHFinishThreads + tid) * 4;
+    f32x4 p;
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+      p[i] = hot ? (e + i == hot_i ? 1.0f : 0.0f)
+                 : __builtin_amdgcn_exp2f((scaled(a, v[k][i]) - M) * kHLog2e) * inv;
+    if (e < a.V) store_logits4(row, e, a.V, p, a.vec_out);
   }
 }
 
@@ -511,10 +694,10 @@ static int head_args(const void *x, int64_t x_stride, const void *w, int64_t w_s
 static int batch_steps(int steps) { return steps == 18 ? 9 : 8; }
 
 // k-steps per staged chunk: the hidden rows of a pass (16 * NCT of them)
-// in at most kHXElems elements, a multiple of kb steps (the last chunk may
+// in at most `elems` elements, a multiple of kb steps (the last chunk may
 // be shorter; it is padded with zeros up to the next multiple)
-static int chunk_steps(int steps, int nct, int kb) {
-  const int row = kHXElems / (kHT * nct);  // elements per staged row
+static int chunk_steps(int steps, int nct, int kb, int elems = kHXElems) {
+  const int row = elems / (kHT * nct);  // elements per staged row
   const int kc = (row - kHXPad) / 32 / kb * kb;
   return std::min((steps + kb - 1) / kb * kb, kc);
 }
@@ -529,6 +712,39 @@ SPECDEC_API int specdec_head_workspace(int64_t *bytes) {
   return SPECDEC_OK;
 }
 
+namespace specdec {
+
+static int launch_head_logits(HeadArgs &a, const HeadPlan &pl, int64_t rows, float *stats, hipStream_t s) {
+  a.tpw = pl.tpw;
+  a.mode = kLogits;
+  a.vec_logits = a.logits_stride % 4 == 0 && ((uintptr_t)a.logits & 15) == 0;
+  // passes of at most four column tiles over the head, as even as they come
+  const int64_t cts = (rows + kHT - 1) / kHT, passes = (cts + 3) / 4;
+  const int nct = (int)((cts + passes - 1) / passes);
+  const int kb = pl.tpw > 12 ? 8 : batch_steps(a.steps);
+  a.kc = chunk_steps(a.steps, nct, kb, nct == 1 ? kHXElems : kHXWide);
+  const int64_t blocks = (int64_t)(pl.grid + 7) / 8 * 8 * passes;
+  if (passes > 65535 || blocks > INT32_MAX) return SPECDEC_EUNSUPPORTED;
+  dim3 grid((unsigned)blocks), block((unsigned)(64 * pl.tpw));
+  const size_t lds = (size_t)kHT * nct * (a.kc * 32 + kHXPad) * 2;
+  const HeadStats hs{stats, pl.grid};
+  const int np = (int)passes;
+#define SPECDEC_HEAD(NCT)                                                                      \
+  do {                                                                                         \
+    if (pl.tpw > 12) head_logits_kernel<NCT, 8, 1024><<<grid, block, lds, s>>>(a, hs, np);  \
+    else if (kb == 9) head_logits_kernel<NCT, 9, 768><<<grid, block, lds, s>>>(a, hs, np);  \
+    else head_logits_kernel<NCT, 8, 768><<<grid, block, lds, s>>>(a, hs, np);               \
+  } while (0)
+  if (nct == 1) SPECDEC_HEAD(1);
+  else if (nct == 2) SPECDEC_HEAD(2);
+  else if (nct == 3) SPECDEC_HEAD(3);
+  else SPECDEC_HEAD(4);
+#undef SPECDEC_HEAD
+  return launch_status();
+}
+
+}  // namespace specdec
+
 SPECDEC_API int specdec_head_logits(const void *x, int64_t x_stride, const void *w, int64_t w_stride, int64_t rows,
                                     int64_t hidden, int64_t vocab, float *logits, int64_t logits_stride,
                                     void *stream) {
@@ -539,27 +755,44 @@ SPECDEC_API int specdec_head_logits(const void *x, int64_t x_stride, const void 
   if (!logits || logits_stride < vocab) return SPECDEC_EINVAL;
   HeadPlan pl;
   if (!plan_head(vocab, false, pl)) return SPECDEC_EUNSUPPORTED;
-  a.tpw = pl.tpw;
-  a.mode = kLogits;
   a.logits = logits;
   a.logits_stride = logits_stride;
-  a.vec_logits = logits_stride % 4 == 0 && ((uintptr_t)logits & 15) == 0;
-  const int nct = rows <= 16 ? 1 : rows <= 32 ? 2 : 4;
-  const int kb = batch_steps(a.steps);
-  a.kc = chunk_steps(a.steps, nct, kb);
-  const int64_t passes = (rows + kHT * nct - 1) / (kHT * nct);
-  if (passes > 65535) return SPECDEC_EUNSUPPORTED;
-  dim3 grid((unsigned)pl.grid, (unsigned)passes), block((unsigned)(64 * pl.tpw));
-  hipStream_t s = as_stream(stream);
-  if (kb == 9) {
-    if (nct == 1) head_logits_kernel<1, 9><<<grid, block, 0, s>>>(a);
-    else if (nct == 2) head_logits_kernel<2, 9><<<grid, block, 0, s>>>(a);
-    else head_logits_kernel<4, 9><<<grid, block, 0, s>>>(a);
-  } else {
-    if (nct == 1) head_logits_kernel<1, 8><<<grid, block, 0, s>>>(a);
-    else if (nct == 2) head_logits_kernel<2, 8><<<grid, block, 0, s>>>(a);
-    else head_logits_kernel<4, 8><<<grid, block, 0, s>>>(a);
-  }
+  return launch_head_logits(a, pl, rows, nullptr, as_stream(stream));
+}
+
+SPECDEC_API int specdec_head_softmax_workspace(int64_t rows, int64_t vocab, int64_t *floats) {
+  if (!floats || rows < 0 || vocab <= 0) return SPECDEC_EINVAL;
+  // a pair per row and slice; a slice holds at least one 16-row tile
+  *floats = 2 * rows * ((vocab + kHT - 1) / kHT);
+  HeadPlan pl;
+  if (plan_head(vocab, false, pl)) *floats = 2 * rows * pl.grid;
+  return SPECDEC_OK;
+}
+
+SPECDEC_API int specdec_head_softmax(const void *x, int64_t x_stride, const void *w, int64_t w_stride, int64_t rows,
+                                     int64_t hidden, int64_t vocab, float temperature, float *out,
+                                     int64_t out_stride, int64_t *index_out, int64_t index_stride, float *workspace,
+                                     int64_t workspace_floats, void *stream) {
+  HeadArgs a;
+  const int st = head_args(x, x_stride, w, w_stride, rows, hidden, vocab, a);
+  if (st != SPECDEC_OK) return st;
+  if (!(temperature >= 0.0f)) return SPECDEC_EINVAL;
+  if (rows == 0) return SPECDEC_OK;
+  if (rows > 65535) return SPECDEC_EUNSUPPORTED;
+  if (!out || out_stride < vocab) return SPECDEC_EINVAL;
+  HeadPlan pl;
+  if (!plan_head(vocab, false, pl)) return SPECDEC_EUNSUPPORTED;
+  if (!workspace || workspace_floats < 2 * rows * pl.grid || ((uintptr_t)workspace & 7)) return SPECDEC_EINVAL;
+  a.temperature = temperature;
+  a.out = a.logits = out;
+  a.out_stride = a.logits_stride = out_stride;
+  a.index_out = temperature == 0.0f ? index_out : nullptr;
+  a.index_stride = index_stride;
+  a.vec_out = out_stride % 4 == 0 && ((uintptr_t)out & 15) == 0;
+  const int s1 = launch_head_logits(a, pl, rows, workspace, as_stream(stream));
+  if (s1 != SPECDEC_OK) return s1;
+  const dim3 grid((unsigned)((vocab + kHFinish - 1) / kHFinish), (unsigned)rows);
+  head_finish_kernel<<<grid, kHFinishThreads, 0, as_stream(stream)>>>(a, HeadStats{workspace, pl.grid});
   return launch_status();
 }
 

@@ -443,6 +443,35 @@ def head_probabilities(x: torch.Tensor, w: torch.Tensor, temperature: float, out
     return o2.view(*x.shape[:-1], v) if fresh else out
 
 
+def head_softmax(x: torch.Tensor, w: torch.Tensor, temperature: float, out: torch.Tensor | None = None,
+                 index_out: torch.Tensor | None = None) -> torch.Tensor:
+    """probabilities(head_logits(x, w), temperature) for any number of rows,
+    in two launches that keep the logits in `out`: fp32 [..., V].  `out` and
+    `index_out` as in head_probabilities."""
+    import ctypes
+
+    x2, rows = _head_operands(x, w)
+    v = w.shape[0]
+    fresh = out is None
+    o2 = _rows_out(out, rows, v, w.device, "out")
+    idx_ptr, idx_stride = None, 0
+    if index_out is not None:
+        if temperature != 0.0:
+            raise ValueError("index_out is defined at temperature 0 only")
+        _on(w.device, index_out, "index_out", torch.int64, numel=rows)
+        if index_out.dim() > 1 and not index_out.is_contiguous():
+            raise ValueError("index_out must be a vector or contiguous")
+        idx_ptr, idx_stride = index_out.data_ptr(), (index_out.stride(0) if index_out.dim() else 1)
+    floats = ctypes.c_int64()
+    _check(lib().specdec_head_softmax_workspace(rows, v, ctypes.byref(floats)), "head_softmax_workspace")
+    ws = torch.empty(floats.value, dtype=torch.float32, device=w.device)
+    st = lib().specdec_head_softmax(x2.data_ptr(), x2.stride(0), w.data_ptr(), w.shape[1], rows, w.shape[1], v,
+                                    float(temperature), o2.data_ptr(), o2.stride(0), idx_ptr, idx_stride,
+                                    ws.data_ptr(), ws.numel(), stream())
+    _check(st, "head_softmax")
+    return o2.view(*x.shape[:-1], v) if fresh else out
+
+
 def head_fused(w: torch.Tensor, rows: int, fastest: bool = False) -> bool:
     """Whether head_probabilities takes `rows` hidden rows against head w on
     this GPU (bf16, H a multiple of 32 up to 2048, the vocab spread over at

@@ -185,3 +185,45 @@ def test_unsupported_shapes_are_refused():
     x, w = operands(2, 48, 1000, seed=1)  # hidden not a multiple of 32
     with pytest.raises(NotImplementedError):
         ops.head_logits(x.to(DEV), w.to(DEV))
+
+
+# one to four column tiles a pass, even and uneven passes, a chunked hidden
+# size, vocabularies that end inside a tile, a slice or a finishing workgroup
+@pytest.mark.parametrize("rows,hidden,vocab", [(1, 2048, 49152), (17, 2048, 4099), (40, 2048, 3001), (64, 2048, 5003),
+                                               (72, 576, 2053), (130, 64, 999), (3, 96, 33), (5, 64, 70001)])
+def test_head_softmax_matches_fp64_and_every_row_alone(rows, hidden, vocab):
+    x, w = operands(rows, hidden, vocab, seed=rows + 7, scale=2.0)
+    xd, wd = x.to(DEV), w.to(DEV)
+    exact = exact_logits(x, w)
+    for temperature in (1.0, 0.8):
+        wide = torch.full((rows, vocab + 5), 7.0, device=DEV)  # rows of a wider tensor, unaligned
+        got = ops.head_softmax(xd, wd, temperature, out=wide[:, 1:vocab + 1])
+        want = torch.softmax(exact / temperature, dim=-1)
+        assert ((got.cpu().double() - want).abs() / want).max().item() < 1e-5
+        assert bool((wide[:, 0] == 7).all()) and bool((wide[:, vocab + 1:] == 7).all())
+        assert torch.equal(got, ops.head_softmax(xd, wd, temperature))
+        for r in sorted({0, rows // 2, rows - 1}):
+            assert torch.equal(ops.head_softmax(xd[r:r + 1], wd, temperature), got[r:r + 1]), r
+    # temperature 0: the lowest id among planted ties
+    w2 = w.clone()
+    for r, t in enumerate(ops.head_logits(xd, wd).argmax(-1).tolist()):
+        w2[(t + 1 + 97 * r) % vocab] = w[t]
+    wd2 = w2.to(DEV)
+    lg = ops.head_logits(xd, wd2)
+    want_idx = torch.tensor([int((lg[r] == lg[r].max()).nonzero()[0]) for r in range(rows)])
+    idx = torch.full((rows, 2), -1, dtype=torch.int64, device=DEV)
+    p = ops.head_softmax(xd, wd2, 0.0, index_out=idx[:, 0])
+    assert torch.equal(idx[:, 0].cpu(), want_idx) and bool((idx[:, 1] == -1).all())
+    assert torch.equal(p.cpu(), torch.nn.functional.one_hot(want_idx, vocab).float())
+
+
+def test_head_softmax_rows_without_a_maximum():
+    """NaN hidden rows give NaN probabilities and an id inside the vocabulary; the other rows are untouched."""
+    x, w = operands(3, 64, 1000, seed=2)
+    x[1] = float("nan")
+    xd, wd = x.to(DEV), w.to(DEV)
+    p = ops.head_softmax(xd, wd, 1.0)
+    assert bool(torch.isnan(p[1]).all()) and torch.equal(p[::2], ops.head_softmax(xd[::2].contiguous(), wd, 1.0))
+    idx = torch.full((3,), -1, dtype=torch.int64, device=DEV)
+    ops.head_softmax(xd, wd, 0.0, index_out=idx)
+    assert 0 <= int(idx[1]) < 1000 and int(idx[0]) == int(ops.head_logits(xd[:1], wd).argmax())
