@@ -218,6 +218,11 @@ __device__ __forceinline__ void store_row4(const AttnArgs &a, const TileInfo &ti
   for (int i = 0; i < 4; ++i) dst[i] = from_f32<T>(v[i]);
 }
 
+// Four floats at an address of their own alignment (4 bytes: q rows and pools
+// come as the caller has them).
+typedef f32x4 __attribute__((aligned(4))) f32x4_any;
+__device__ __forceinline__ f32x4 load4(const float *p) { return *reinterpret_cast<const f32x4_any *>(p); }
+
 // A row whose cached length exceeds the call's max_kv_len (a caller broke
 // the contract): its tile's output rows are set to NaN by the tile's first
 // workgroup, so the error shows instead of stale output.
@@ -1597,7 +1602,7 @@ __global__ __launch_bounds__(kPThreads) __attribute__((amdgpu_waves_per_eu(3))) 
 // ---------------------------------------------------------------- fp32 ----
 // Same structure on v_mfma_f32_16x16x4_f32: per 16-token group the k index
 // of lane group g is dim 16g+s at step s (QK^T) and token 4g+i at step i (PV).
-template <bool BS16>
+// Block sizes that are not a multiple of 16.
 __global__ __launch_bounds__(kAttnThreads) void attention_f32_kernel(AttnArgs a) {
   TileInfo ti;
   if (!tile_info(a, ti)) {
@@ -1664,16 +1669,16 @@ __global__ __launch_bounds__(kAttnThreads) void attention_f32_kernel(AttnArgs a)
         for (int i = 0; i < 4; ++i) vv[gi][tt][i] = 0.0f;
       if (gs < ti.kv_len) {
         const int pos = gs + c;
-        if (BS16 || pos < ti.kv_len) {
-          const int64_t blk = block_of(a, ti, BS16 ? gs : pos);
-          const float *kb = kp + ((blk * Hkv + ti.h) * bs + (BS16 ? gs % bs + c : pos % bs)) * kD + 16 * g;
+        if (pos < ti.kv_len) {
+          const int64_t blk = block_of(a, ti, pos);
+          const float *kb = kp + ((blk * Hkv + ti.h) * bs + pos % bs) * kD + 16 * g;
 #pragma unroll
           for (int s = 0; s < 16; ++s) kv[s] = kb[s];
         }
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
           const int vpos = gs + 4 * g + i;
-          const bool ok = BS16 || vpos < ti.kv_len;
+          const bool ok = vpos < ti.kv_len;
           const int64_t blk = ok ? block_of(a, ti, vpos) : 0;
           const float *vb = vp + (blk * Hkv + ti.h) * (int64_t)kD * bs + vpos % bs;
 #pragma unroll
@@ -1698,6 +1703,139 @@ __global__ __launch_bounds__(kAttnThreads) void attention_f32_kernel(AttnArgs a)
 #pragma unroll
         for (int i = 0; i < 4; ++i)
           o[tt] = __builtin_amdgcn_mfma_f32_16x16x4f32(vv[gi][tt][i], sv[4 * gi + i], o[tt], 0, 0, 0);
+  }
+  finish<float>(a, ti, m, l, o);
+}
+
+// Block sizes that are a multiple of 16.  A call reads a few MB through a
+// grid of a few hundred workgroups, so the waves' dependent round trips bound
+// it: each 16-token group's block id, then its K and V, four times per wave
+// one after another, took 32 us for 4 rows of 1024 keys (34 MB); this kernel 16.5.
+// A wave holds a
+// 64-token step as two 32-token chunks whose loads are all in flight, the
+// block ids a step ahead, and a chunk's registers are loaded again for the
+// next step as soon as it is multiplied.  The k index of lane group g at step
+// 4 j + i is dim 16 j + 4 g + i, so a K load reads 64 consecutive bytes of
+// each of 16 tokens and RoPE's partner (32 dims away) is in the same lane; a V
+// load reads a contiguous KB of the dim-major tile at 16-token blocks.
+__global__ __launch_bounds__(kAttnThreads) __attribute__((amdgpu_waves_per_eu(2, 2))) void
+attention_f32_groups_kernel(AttnArgs a) {
+  TileInfo ti;
+  tile_coords(a, blockIdx.x, ti);
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int g = lane >> 4, c = lane & 15;
+  // this lane's query row: dims 16 j + 4 g .. of its head, before the metadata
+  // (rows past the row's new tokens are dropped below)
+  const int r = ti.qt * kRows + c, rq = min(r, a.width * ti.group - 1);
+  const float *qrow = reinterpret_cast<const float *>(a.q) + ((int64_t)ti.b * a.width + rq / ti.group) * a.q_stride +
+                      (int64_t)(ti.h * ti.group + rq % ti.group) * kD + 4 * g;
+  f32x4 qv[4];
+#pragma unroll
+  for (int j = 0; j < 4; ++j) qv[j] = load4(qrow + 16 * j);
+  if (!tile_meta(a, ti, /*any_split=*/false)) {
+    poison_tile<float>(a, ti);
+    return;
+  }
+  const bool row_ok = r < ti.nrows;
+  const int qpos = ti.past + (row_ok ? r / ti.group : 0);
+  const int s_lo = blockIdx.y * a.split, s_hi = min(s_lo + a.split, ti.kv_len);
+  const int bs = a.bs, last_blk = (ti.kv_len - 1) / bs;
+  const int32_t *trow = a.tables + (int64_t)ti.row * a.table_stride;
+  const int64_t tile_elems = (int64_t)bs * kD;
+  const float *kp = reinterpret_cast<const float *>(a.k), *vp = reinterpret_cast<const float *>(a.v);
+  // block ids of the step at c0 (lane j & 3: tokens c0 + 16j ..)
+  auto step_blocks = [&](int c0) -> int { return trow[min((c0 + 16 * (lane & 3)) / bs, last_blk)]; };
+  const int first = s_lo + 64 * wave;
+  int bj = step_blocks(first), bn = step_blocks(first + 256);
+  if (a.rope) {
+    f32x4 cs[2], sn[2];
+#pragma unroll
+    for (int j = 0; j < 2; ++j) {
+      cs[j] = load4(a.cos_t + (int64_t)qpos * (kD / 2) + 16 * j + 4 * g);
+      sn[j] = load4(a.sin_t + (int64_t)qpos * (kD / 2) + 16 * j + 4 * g);
+    }
+#pragma unroll
+    for (int j = 0; j < 2; ++j)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        float y1, y2;
+        rope_pair(qv[j][i], qv[j + 2][i], cs[j][i], sn[j][i], y1, y2);
+        qv[j][i] = y1;
+        qv[j + 2][i] = y2;
+      }
+    append_new_kv<float>(a, ti, s_lo, s_lo + a.split);
+    __threadfence_block();
+    __syncthreads();
+  }
+  const float c2 = a.scale * 1.4426950408889634f;  // scores in log2 units
+
+  f32x4 o[4];
+#pragma unroll
+  for (int tt = 0; tt < 4; ++tt) o[tt] = f32x4{0.f, 0.f, 0.f, 0.f};
+  float m = -INFINITY, l = 0.0f;
+  struct Chunk {
+    f32x4 k[2][4], v[2][4];  // [16-token group][..]
+  };
+  // chunk ch (0, 1) of the step at c0; a group past the keys reads the row's
+  // last block, and its scores are masked
+  auto issue = [&](Chunk &x, int c0, int ch, int bjv) {
+#pragma unroll
+    for (int gi = 0; gi < 2; ++gi) {
+      const int64_t tile = ((int64_t)__builtin_amdgcn_readlane(bjv, 2 * ch + gi) * a.Hkv + ti.h) * tile_elems;
+      const int in = (c0 + 32 * ch + 16 * gi) % bs;
+      const float *kb = kp + tile + (int64_t)(in + c) * kD + 4 * g, *vb = vp + tile + (int64_t)c * bs + in + 4 * g;
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        x.k[gi][j] = load4(kb + 16 * j);
+        x.v[gi][j] = load4(vb + (int64_t)16 * j * bs);
+      }
+    }
+  };
+  auto compute = [&](const Chunk &x, int cs) {
+    if (cs >= s_hi) return;
+    float sv[8];
+#pragma unroll
+    for (int gi = 0; gi < 2; ++gi) {
+      f32x4 s4 = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int j = 0; j < 4; ++j)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) s4 = __builtin_amdgcn_mfma_f32_16x16x4f32(x.k[gi][j][i], qv[j][i], s4, 0, 0, 0);
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const int pos = cs + 16 * gi + 4 * g + i;
+        sv[4 * gi + i] = row_ok && pos <= qpos && pos < ti.kv_len ? s4[i] * c2 : -INFINITY;
+      }
+    }
+    online_update(sv, m, l, o);
+#pragma unroll
+    for (int gi = 0; gi < 2; ++gi)
+#pragma unroll
+      for (int tt = 0; tt < 4; ++tt)
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+          o[tt] = __builtin_amdgcn_mfma_f32_16x16x4f32(x.v[gi][tt][i], sv[4 * gi + i], o[tt], 0, 0, 0);
+  };
+  // wave w takes the 64-token steps w, w + 4, ... of this split
+  if (first < s_hi) {
+    Chunk x0, x1;
+    issue(x0, first, 0, bj);
+    issue(x1, first, 1, bj);
+    int c0 = first;
+    for (; c0 + 256 < s_hi; c0 += 256) {
+      bj = bn;
+      bn = step_blocks(c0 + 512);
+      compute(x0, c0);
+      __builtin_amdgcn_sched_barrier(0);
+      issue(x0, c0 + 256, 0, bj);
+      __builtin_amdgcn_sched_barrier(0);
+      compute(x1, c0 + 32);
+      __builtin_amdgcn_sched_barrier(0);
+      issue(x1, c0 + 256, 1, bj);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+    compute(x0, c0);
+    compute(x1, c0 + 32);
   }
   finish<float>(a, ti, m, l, o);
 }
@@ -1892,8 +2030,8 @@ static int run_attention(AttnArgs &a, const AttnPlan &plan, int dtype, int32_t b
     else attention_bf16_kernel<0, 4><<<grid, block, 0, s>>>(a);
   } else {
     dim3 block(kAttnThreads);
-    if (bs16) attention_f32_kernel<true><<<grid, block, 0, s>>>(a);
-    else attention_f32_kernel<false><<<grid, block, 0, s>>>(a);
+    if (bs16) attention_f32_groups_kernel<<<grid, block, 0, s>>>(a);
+    else attention_f32_kernel<<<grid, block, 0, s>>>(a);
   }
   if (a.parts > 1) {
     dim3 cg((unsigned)units), cb(kAttnThreads);

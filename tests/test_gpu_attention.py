@@ -869,3 +869,12 @@ def test_prefill_rows_do_not_depend_on_the_batch_and_scales_of_any_sign():
         for b in range(3):
             assert torch.equal(call([b], scale), together[b:b + 1]), (scale, b)
             assert (got[b, :, :t_new[b]] - want[b, :, :t_new[b]]).abs().max().item() < 2e-2, (scale, b)
+
+
+@pytest.mark.parametrize("lengths,heads,bs", [([31, 63, 64, 255], (4, 4), 16), ([256, 257, 507, 513], (9, 3), 48),
+                                              ([769, 1020, 1, 16], (16, 1), 32)])
+def test_fp32_step_and_split_edges_match_oracle(lengths, heads, bs):
+    """Contexts that end at the edges of a wave's 32-token chunks and 64-token
+    steps and of the 512-token splits, blocks of 16, 32 and 48."""
+    for got, want in run_case(len(lengths), lengths, *heads, bs, torch.float32, 5, seed=bs):
+        assert (got - want).abs().max().item() < 2e-5
