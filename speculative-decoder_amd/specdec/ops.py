@@ -805,11 +805,18 @@ def linear_attn_parts(parts: torch.Tensor, rows: int, n_heads: int, w: torch.Ten
 
 def latency_split(batch: int, width: int, n_heads: int, n_kv_heads: int, max_kv_len: int) -> int:
     """A split for calls whose bits need not match any other call (the draft
-    model).  With few (row, head) units: -1, one 16-wave workgroup per unit
-    striding every key, so no combine kernel is launched; otherwise 0 (the
-    default)."""
+    model).  Up to 2048 keys: -1, one workgroup per (row, head) unit striding
+    every key, so no combine kernel is launched, for one-token rows and for few
+    units, else 0 (the default).  Measured at the draft's heads, 64 rows: 7.1
+    us at 300 keys and 13.6 at 1000 against 10.3 and 14.7 with the default
+    (32 rows at 2000: 18.6 against 17.7).  Past 2048 keys one workgroup per
+    unit takes a microsecond for each 170 keys (one row of 4000: 25.6 us), so
+    the keys are split: by 256 while that gives at most four workgroups per
+    compute unit (10.9 us), else by 512 (32 rows of 2500: 18.0 against 19.9)."""
     units = batch * n_kv_heads * -(-(width * (n_heads // n_kv_heads)) // 16)
-    return -1 if units < 64 else 0
+    if max_kv_len <= 2048:
+        return -1 if units < 64 or width == 1 else 0
+    return 256 if units * -(-max_kv_len // 256) <= 1024 else 512
 
 
 def _qkv_side(dev, x, cos, sin, meta, batch, width, tables, k_pool, v_pool, out=None) -> None:

@@ -878,3 +878,34 @@ def test_fp32_step_and_split_edges_match_oracle(lengths, heads, bs):
     steps and of the 512-token splits, blocks of 16, 32 and 48."""
     for got, want in run_case(len(lengths), lengths, *heads, bs, torch.float32, 5, seed=bs):
         assert (got - want).abs().max().item() < 2e-5
+
+
+@pytest.mark.parametrize("batch,length,want", [(1, 2040, -1), (30, 100, -1), (1, 2100, 256), (8, 4000, 256),
+                                               (32, 2500, 512)])
+def test_latency_split_follows_the_keys_and_matches_the_default(batch, length, want):
+    """The draft's split: one workgroup per unit up to 2048 keys, 256- or
+    512-token splits past them; the rows agree with the default split's to
+    bf16 rounding."""
+    h, hkv, d, bs = 9, 3, 64, 16
+    max_kv = 2048 if length < 2048 else 4096
+    split = ops.latency_split(batch, 1, h, hkv, max_kv)
+    assert split == want
+    g = torch.Generator(device="cuda").manual_seed(batch)
+    cache = KVCache(1, hkv, d, batch * (length // bs + 2), bs, torch.bfloat16, "cuda")
+    ids = list(range(batch))
+    for s in ids:
+        cache.add(s)
+    step = cache.append(ids, [length] * batch)
+    k, v = (torch.randn(batch, hkv, length, d, generator=g, device="cuda").to(torch.bfloat16) for _ in range(2))
+    cache.write(0, step, k, v)
+    step = cache.append(ids, [1] * batch)
+    qkv = torch.randn(batch, 1, (h + 2 * hkv) * d, generator=g, device="cuda").to(torch.bfloat16)
+    cos, sin = torch.ones(4097, d // 2, device="cuda"), torch.zeros(4097, d // 2, device="cuda")
+    outs = []
+    for sp in (split, 0):
+        out = torch.zeros(batch, 1, h * d, dtype=torch.bfloat16, device="cuda")
+        ops.rope_paged_attention(qkv, cos, sin, cache.k[0], cache.v[0], cache.table_tensor, step.meta, batch, 1, h,
+                                 hkv, d, bs, 0.125, max_kv, out, out.stride(1), split_tokens=sp)
+        outs.append(out.float())
+    # a bf16 step of values below 1, and the weights' rounding to bf16
+    assert (outs[0] - outs[1]).abs().max().item() < 1e-2
