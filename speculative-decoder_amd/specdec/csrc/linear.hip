@@ -18,7 +18,7 @@
 // k = 32s + 8g; B = x rows, the same layout, rows past M reading zeros
 // through the buffer bound).  The waves' partial sums meet in LDS and are
 // added in wave order; lane (c, g) then holds row c's features 4g .. 4g+3.
-// More than 16 rows: linear_rows_kernel, several 16-row column tiles per wave
+// More rows: linear_rows_kernel, several 16-row column tiles per wave
 // with x through LDS.
 // Each output element goes through the same operations whatever M is, so
 // a row's result does not depend on the other rows of the call: a token
@@ -74,13 +74,18 @@ __device__ __forceinline__ void w_lane(const LinArgs &a, int tile, int row, int 
   }
 }
 
-// At most 16 rows; KB k-steps per load batch.
-template <int KB>
+// At most 16 rows; KB k-steps per load batch.  PART workgroups per feature
+// tile (weights with fewer tiles than compute units): each reads and stores
+// 16 / PART of the tile's features, the other lanes' W operands read out of
+// range (zeros); an output's operations are the same.
+template <int KB, int PART>
 __global__ __launch_bounds__(kLinMaxWaves * 64) void linear_kernel(LinArgs a) {
   __shared__ f32x4 s_acc[kLinMaxWaves][64];
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, nw = blockDim.x >> 6;
   const int c = lane & 15, g = lane >> 4;
-  const int n0 = blockIdx.x * 16;
+  const int tile = PART == 1 ? blockIdx.x : blockIdx.x / PART;
+  const int n0 = tile * 16, part = PART == 1 ? 0 : blockIdx.x % PART;
+  const bool mine = PART == 1 || c / (16 / PART) == part;
   const int s_lo = wave * a.per_wave;
   const int cnt = max(min(a.per_wave, a.steps - s_lo), 0);
   // W rows past N read the last row (never stored); x rows past M read zeros
@@ -90,7 +95,7 @@ __global__ __launch_bounds__(kLinMaxWaves * 64) void linear_kernel(LinArgs a) {
       const_cast<uint16_t *>(a.x), 0, (int)(((int64_t)(a.M - 1) * a.x_stride + a.K) * 2), 0x00020000);
   const int row = min(n0 + c, a.N - 1);
   unsigned wbase, wstep;
-  w_lane(a, blockIdx.x, row, lane, wbase, wstep);
+  w_lane(a, tile, row, lane, wbase, wstep);
   const unsigned xbase = (unsigned)(((int64_t)c * a.x_stride + 8 * g) * 2);
   // accumulate: the values added before the rounding, loaded now so their
   // round trip overlaps the weight's
@@ -117,7 +122,7 @@ __global__ __launch_bounds__(kLinMaxWaves * 64) void linear_kernel(LinArgs a) {
 #pragma unroll
     for (int j = 0; j < KB; ++j) {
       const unsigned s = (unsigned)(s_lo + min(b * KB + j, cnt - 1));
-      A[j] = __builtin_amdgcn_raw_buffer_load_b128(wb, wbase + s * wstep, 0, 0);
+      A[j] = __builtin_amdgcn_raw_buffer_load_b128(wb, mine ? wbase + s * wstep : 0xFFFFFF00u, 0, 0);
       B[j] = __builtin_amdgcn_raw_buffer_load_b128(xb, xbase + s * 64u, 0, 0);
     }
   };
@@ -156,7 +161,7 @@ __global__ __launch_bounds__(kLinMaxWaves * 64) void linear_kernel(LinArgs a) {
   s_acc[wave][lane] = acc;
   __syncthreads();
   // the sums of the waves, in wave order
-  if (wave == 0 && c < a.M) {
+  if (wave == 0 && c < a.M && (PART == 1 || 4 * g / (16 / PART) == part)) {
     f32x4 t = s_acc[0][lane];
     for (int w = 1; w < nw; ++w) t += s_acc[w][lane];
     uint16_t *dst = a.out + (int64_t)c * a.out_stride + f0;
@@ -448,7 +453,7 @@ __global__ __launch_bounds__(kLinMaxWaves * 64) void linear_silu_kernel(LinArgs 
   }
 }
 
-// 17 to 64 rows: the same sums in the same order as linear_kernel's and
+// Up to 64 rows: the same sums in the same order as linear_kernel's and
 // linear_silu_kernel's (one k-split, the waves' sums folded in wave order),
 // so a row's bits do not depend on which of them ran.
 //
@@ -663,7 +668,7 @@ __global__ __launch_bounds__(kLinMaxWaves * 64) void linear_rows_kernel(LinArgs 
   }
 }
 
-// The gate/up form for 17 to 64 rows (linear_silu_kernel's sums and
+// The gate/up form (linear_silu_kernel's sums and
 // epilogue): NP gate tiles and their up tiles per workgroup, the rows' norm
 // scales computed along the chunks (RowScales).
 template <int NCT, int NP, int RS, int NVH, int Q, int TH>
@@ -820,8 +825,19 @@ SPECDEC_API int specdec_linear(const void *x, int64_t x_stride, const void *w, i
   linear_split(a, tiles, waves);
   const dim3 grid((unsigned)tiles), block((unsigned)(64 * waves));
   hipStream_t s = as_stream(stream);
+  const int cus = std::max(cu_count(), 1);
   if (rows <= 16) {
-    linear_kernel<8><<<grid, block, 0, s>>>(a);
+    // From 9 rows x outweighs W's latency where every compute unit has a tile:
+    // two tiles share x through LDS (1.7B qkv, 16 rows: 8.1 against 9.5 us; 5
+    // rows 7.7 against 7.6).  With less than half a tile for each, two
+    // workgroups take a tile's features (1.7B down, 5 rows: 11.1 against 12.7
+    // us, o 5.1 against 5.4, draft down 3.6 against 3.7); a short projection
+    // gains nothing once x weighs in (draft down, 9 rows: 4.1 against 3.9) or
+    // without the residual (draft qkv, 5 rows: 2.87 against 2.79).
+    if (rows > 8 && tiles >= cus) launch_linear_rows<1, 2, 4>(a, tiles, waves, s);
+    else if (2 * tiles <= cus && (a.steps >= 64 || (a.accumulate && rows <= 8)))
+      linear_kernel<8, 2><<<dim3((unsigned)(2 * tiles)), block, 0, s>>>(a);
+    else linear_kernel<8, 1><<<grid, block, 0, s>>>(a);
     return launch_status();
   }
   // 17 to 64 rows.  Few feature tiles: column tiles go to workgroups of their
@@ -829,7 +845,7 @@ SPECDEC_API int specdec_linear(const void *x, int64_t x_stride, const void *w, i
   // rows: 16.1 us as two workgroups of two column tiles, 23.1 as one of four,
   // 19.3 as four of one).  A tile for every compute unit and more: two tiles a
   // workgroup (qkv, 384 tiles, 64 rows: 10.6 against 14.5 us).
-  const int ct = (int)((rows + 15) / 16), cus = std::max(cu_count(), 1);
+  const int ct = (int)((rows + 15) / 16);
   const int groups = (int)std::min<int64_t>(ct, std::max<int64_t>(1, cus / tiles));
   const int nct = (ct + groups - 1) / groups;
   if (tiles >= cus) {
@@ -929,23 +945,24 @@ SPECDEC_API int specdec_linear_silu(const void *x, int64_t x_stride, const void 
   const int hd = (int)hidden_dim, nvec = hd / 8;
   hipStream_t s = as_stream(stream);
   // (linear_silu_rows_kernel addresses the residual rows by 32-bit offsets)
-  if (rows > 16 && rows * hidden_stride * 2 > INT32_MAX) {
-    for (int64_t r = 0; r < rows; r += 16) {
+  if (rows > 12 && rows * hidden_stride * 2 > INT32_MAX) {
+    for (int64_t r = 0; r < rows; r += 12) {
       const int st = specdec_linear_silu(a.x + r * x_stride, x_stride, w, w_stride, w_layout,
-                                         std::min<int64_t>(16, rows - r), in_features, inter, h + r * hidden_stride,
+                                         std::min<int64_t>(12, rows - r), in_features, inter, h + r * hidden_stride,
                                          hidden_stride, hidden_dim, eps, a.out + r * out_stride, out_stride, stream);
       if (st != SPECDEC_OK) return st;
     }
     return SPECDEC_OK;
   }
-  if (rows <= 16) {
+  if (rows <= 12) {
     if (nvec <= 2 * 64) linear_silu_kernel<4, 2><<<grid, block, 0, s>>>(a, h, hidden_stride, hd, eps, (int)inter);
     else if (nvec <= 4 * 64) linear_silu_kernel<4, 4><<<grid, block, 0, s>>>(a, h, hidden_stride, hd, eps, (int)inter);
     else linear_silu_kernel<4, 8><<<grid, block, 0, s>>>(a, h, hidden_stride, hd, eps, (int)inter);
     return launch_status();
   }
-  // 17 to 64 rows.  Every workgroup computes the norm scales of its rows, so
-  // with few tiles the column tiles are spread further than the plain
+  // 13 to 64 rows (at 16 the 1.7B's takes 17.0 against 18.3 us, the draft's 5.0
+  // against 5.9, at 9 rows 16.6 and 4.4 either way).  Every workgroup computes
+  // the norm scales of its rows, so with few tiles the column tiles are spread further than the plain
   // projection's (draft, 96 tiles, 32 rows: 5.0 us as one column tile a
   // workgroup, 7.2 as two), and with two tiles for every compute unit a
   // workgroup takes two (1.7B, 40 rows: 20.1 against 24.2 us).
@@ -956,7 +973,8 @@ SPECDEC_API int specdec_linear_silu(const void *x, int64_t x_stride, const void 
 #define SPECDEC_SILU_ROWS(NCT, NP, RS) \
   launch_silu_rows<NCT, NP, RS>(a, waves, h, hidden_stride, hd, eps, (int)inter, s)
   if (tiles >= 2 * cus) {
-    if (nct == 2) SPECDEC_SILU_ROWS(2, 2, 2);
+    if (nct == 1) SPECDEC_SILU_ROWS(1, 2, 2);
+    else if (nct == 2) SPECDEC_SILU_ROWS(2, 2, 2);
     else if (nct == 3) SPECDEC_SILU_ROWS(3, 2, 2);
     else SPECDEC_SILU_ROWS(4, 2, 2);
   } else if (nct == 1) SPECDEC_SILU_ROWS(1, 1, 4);

@@ -183,32 +183,36 @@ def test_linear_silu_tiled_weight_gives_the_same_bits(rows, k, inter):
     assert torch.equal(a, b)
 
 
-# every instance of the 17-64 row kernels and its edges: column tiles to
+# every instance of the kernels for more rows and its edges: column tiles to
 # workgroups of their own (few feature tiles), one workgroup of 3 or 4, two
 # feature tiles a workgroup with an odd count, a ragged k-split, a last chunk
 # of one k-step, rows one past a column tile
 @pytest.mark.parametrize("rows,k,n,tiled", [(17, 576, 960, True), (33, 2048, 2048, True), (49, 96, 3088, True),
                                             (40, 160, 3000, False), (20, 96, 4112, True), (48, 288, 4112, True),
-                                            (64, 2080, 4100, False), (41, 1056, 2208, True), (64, 32, 33, False)])
-def test_more_rows_equal_sixteen_at_a_time_bitwise(rows, k, n, tiled):
+                                            (64, 2080, 4100, False), (41, 1056, 2208, True), (64, 32, 33, False),
+                                            (16, 288, 4112, True), (9, 2048, 4100, False), (8, 576, 576, True),
+                                            (16, 2112, 2048, True)])
+def test_more_rows_equal_few_at_a_time_bitwise(rows, k, n, tiled):
     x, w = operands(rows, k, n, seed=rows + n)
     xd, wd = x.to(DEV), w.to(DEV)
     wd = ops.tile_weight(wd) if tiled else wd
     base = torch.randn(rows, n, generator=torch.Generator().manual_seed(1)).to(torch.bfloat16).to(DEV)
     plain, added = ops.linear(xd, wd), base.clone()
     ops.linear(xd, wd, out=added, accumulate=True)
-    for r in range(0, rows, 16):
-        part = slice(r, min(r + 16, rows))
-        want = base[part].clone()
-        ops.linear(xd[part], wd, out=want, accumulate=True)
-        assert torch.equal(plain[part], ops.linear(xd[part], wd)) and torch.equal(added[part], want), r
+    for few in (16, 7, 1):
+        for r in range(0, rows, few):
+            part = slice(r, min(r + few, rows))
+            want = base[part].clone()
+            ops.linear(xd[part], wd, out=want, accumulate=True)
+            assert torch.equal(plain[part], ops.linear(xd[part], wd)) and torch.equal(added[part], want), (few, r)
 
 
 @pytest.mark.parametrize("rows,k,inter,hdim,tiled", [(17, 576, 1536, 576, True), (33, 96, 4816, 96, True),
                                                      (64, 160, 4800, 160, True), (20, 288, 8208, 288, True),
                                                      (40, 2048, 8208, 2048, True), (64, 544, 8200, 4096, False),
-                                                     (49, 64, 104, 1024, False), (31, 2048, 1040, 4096, False)])
-def test_more_silu_rows_equal_sixteen_at_a_time_bitwise(rows, k, inter, hdim, tiled):
+                                                     (49, 64, 104, 1024, False), (31, 2048, 1040, 4096, False),
+                                                     (16, 288, 8208, 288, True), (13, 576, 1536, 576, True)])
+def test_more_silu_rows_equal_few_at_a_time_bitwise(rows, k, inter, hdim, tiled):
     g = torch.Generator().manual_seed(rows + inter)
     w = (torch.randn(2 * inter, k, generator=g) * 0.05).to(torch.bfloat16).to(DEV)
     w = ops.tile_weight(w) if tiled else w
@@ -218,6 +222,7 @@ def test_more_silu_rows_equal_sixteen_at_a_time_bitwise(rows, k, inter, hdim, ti
     out = torch.full((rows, inter), 7.0, dtype=torch.bfloat16, device=DEV)
     ops.linear_silu(x, w, hidden, out, 1e-5)
     want = torch.empty_like(out)
-    for r in range(0, rows, 16):
-        ops.linear_silu(x[r:r + 16], w, hidden[r:r + 16], want[r:r + 16], 1e-5)
-    assert torch.equal(out, want)
+    for few in (16, 5):
+        for r in range(0, rows, few):
+            ops.linear_silu(x[r:r + few], w, hidden[r:r + few], want[r:r + few], 1e-5)
+        assert torch.equal(out, want), few
