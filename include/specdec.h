@@ -140,6 +140,22 @@ int specdec_accept_reject_logits(const void *target_logits, const void *draft_lo
                                  int64_t *out, void *workspace, int64_t workspace_bytes,
                                  int32_t spin, void *stream);
 
+/* specdec_accept_reject and specdec_accept_reject_logits with the drafted ids
+ * behind the verdict: out [3 + k, batch], rows 3 .. the draft transposed, so
+ * that one copy brings the host all that a round settles. */
+int specdec_accept_verdict(const void *p, const void *q, int dtype, int64_t p_batch_stride,
+                           int64_t p_row_stride, int64_t q_batch_stride, int64_t q_row_stride,
+                           const int64_t *draft, const void *u_accept, const void *u_residual,
+                           int64_t batch, int64_t k, int64_t vocab, int64_t *out, void *workspace,
+                           int64_t workspace_bytes, int32_t spin, void *stream);
+int specdec_accept_verdict_logits(const void *target_logits, const void *draft_logits, int dtype,
+                                  int64_t t_batch_stride, int64_t t_row_stride,
+                                  int64_t d_batch_stride, int64_t d_row_stride, float temperature,
+                                  const int64_t *draft, const void *u_accept,
+                                  const void *u_residual, int64_t batch, int64_t k, int64_t vocab,
+                                  int64_t *out, void *workspace, int64_t workspace_bytes,
+                                  int32_t spin, void *stream);
+
 /* First stage of accept-reject alone (for a caller-supplied residual):
  * out int64 [2, batch]: n_accepted and a flag that is 1 when a drafted token
  * had q(x) <= 0 or an id outside [0, vocab) (such an id is never read

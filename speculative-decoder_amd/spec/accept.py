@@ -71,15 +71,26 @@ _BAD_DRAFT = ("a drafted token has zero draft probability or lies outside the vo
               "was sampled from")
 
 
-def _settle(out: torch.Tensor, draft_d: torch.Tensor) -> Verdict:
-    """The kernel's [3, B] output and the draft brought to the host in one
-    copy; the reference's ValueError for a bad draft."""
-    host = torch.cat([out, draft_d.t()]).cpu()
-    if bool(host[2].any()):
+def _settle(out: torch.Tensor) -> Verdict:
+    """The kernel's [3 + k, B] output (the verdict, then the draft) brought to
+    the host in one copy; the reference's ValueError for a bad draft."""
+    host = out.cpu()
+    if any(host[2].tolist()):
         raise ValueError(_BAD_DRAFT)
-    verdict = Verdict(host[0].clone(), host[1].clone())
+    verdict = Verdict(host[0], host[1])
     object.__setattr__(verdict, "_host_draft", host[3:].t())
     return verdict
+
+
+def _upload_uniforms(u_accept: torch.Tensor, u_residual: torch.Tensor,
+                     dtype: torch.dtype) -> tuple[torch.Tensor, torch.Tensor]:
+    """Both uniforms on the GPU, contiguous, in `dtype`; from the host in one copy."""
+    if u_accept.device.type == "cpu" and u_residual.device.type == "cpu":
+        n, shape = u_accept.numel(), u_accept.shape
+        both = torch.cat([u_accept.reshape(-1).to(dtype), u_residual.reshape(-1).to(dtype)])
+        both = both.to("cuda", non_blocking=True)
+        return both[:n].view(shape), both[n:].view(u_residual.shape)
+    return _cuda(u_accept.to(dtype)).contiguous(), _cuda(u_residual.to(dtype)).contiguous()
 
 
 def _uniforms(shape: tuple[int, ...], generator: torch.Generator | None, dtype: torch.dtype) -> torch.Tensor:
@@ -111,11 +122,10 @@ def accept_reject(
     p = _cuda(p)
     q = _cuda(q.to(p.dtype))
     draft_d = _cuda(draft.to(torch.int64)).contiguous()
-    ua = _cuda(u_accept.to(p.dtype)).contiguous()
-    ur = _cuda(u_residual.to(p.dtype)).contiguous()
+    ua, ur = _upload_uniforms(u_accept, u_residual, p.dtype)
     if residual is residual_distribution:
         # the draft rides in the verdict's one copy to the host
-        return _settle(ops.accept_reject(p, q, draft_d, ua, ur), draft_d)
+        return _settle(ops.accept_reject(p, q, draft_d, ua, ur, with_draft=True))
     stage = ops.accept_count(p, q, draft_d, ua)
     n_host = stage.cpu()
     if bool(n_host[1].any()):
@@ -153,12 +163,11 @@ def accept_reject_logits(
     tl = _cuda(target_logits).float()
     dl = _cuda(draft_logits).float()
     draft_d = _cuda(draft.to(torch.int64)).contiguous()
-    ua = _cuda(u_accept.float()).contiguous()
-    ur = _cuda(u_residual.float()).contiguous()
-    out = ops.accept_reject_logits(tl, dl, temperature, draft_d, ua, ur)
+    ua, ur = _upload_uniforms(u_accept, u_residual, torch.float32)
+    out = ops.accept_reject_logits(tl, dl, temperature, draft_d, ua, ur, with_draft=True)
     if out is None:
         from lm.sampling import probabilities
 
         return accept_reject(probabilities(tl, temperature), probabilities(dl, temperature), draft, u_accept=ua,
                              u_residual=ur)
-    return _settle(out, draft_d)
+    return _settle(out)

@@ -20,6 +20,9 @@ SIGNATURES: dict[str, list] = {
     "specdec_accept_reject": [P, P, c_int, I64, I64, I64, I64, P, P, P, I64, I64, I64, P, P, I64, I32, P],
     "specdec_accept_reject_logits": [P, P, c_int, I64, I64, I64, I64, c_float, P, P, P, I64, I64, I64, P, P, I64,
                                      I32, P],
+    "specdec_accept_verdict": [P, P, c_int, I64, I64, I64, I64, P, P, P, I64, I64, I64, P, P, I64, I32, P],
+    "specdec_accept_verdict_logits": [P, P, c_int, I64, I64, I64, I64, c_float, P, P, P, I64, I64, I64, P, P, I64,
+                                      I32, P],
     "specdec_accept_count": [P, P, c_int, I64, I64, I64, I64, P, P, I64, I64, I64, P, P],
     "specdec_sample_inverse_cdf": [P, c_int, I64, I64, I64, P, P, P],
     "specdec_one_hot": [P, I64, I64, P, P],

@@ -664,6 +664,7 @@ struct MwArgs {
   float temperature;  // logits form
   int spin;
   int64_t *out;
+  int64_t *draft_out;  // the drafted ids, [k, batch], or null
   uint64_t *ws;
 };
 
@@ -1033,6 +1034,9 @@ __global__ __launch_bounds__(kMwThreads) void accept_reject_mw_kernel(MwArgs a) 
   typedef const __attribute__((address_space(4))) uint64_t const_u64;
   typedef const __attribute__((address_space(4))) float const_f32;
   typedef const __attribute__((address_space(4))) int64_t const_i64;
+  // this row's drafted ids for the caller: read now, written with the verdict
+  int64_t id_copy = 0;
+  if (a.draft_out && g == 0 && tid < k) id_copy = a.draft[b * k + tid];
   uint64_t epoch;
   float ur;
   float lt = 0.0f, ld = 0.0f, uacc = 0.0f;  // logits form: position tid's inputs
@@ -1200,6 +1204,10 @@ __global__ __launch_bounds__(kMwThreads) void accept_reject_mw_kernel(MwArgs a) 
     a.out[b] = n;
     a.out[2 * a.batch + b] = bad;
   }
+  if (a.draft_out && g == 0) {
+    if (tid < k) a.draft_out[tid * a.batch + b] = id_copy;
+    for (int64_t t = tid + kMwThreads; t < k; t += kMwThreads) a.draft_out[t * a.batch + b] = a.draft[b * k + t];
+  }
 
   // B: the chunk's residual sum
   float x[E], pv[E];  // this thread's residual elements and p, then the quotients
@@ -1285,6 +1293,14 @@ __global__ void one_hot_kernel(const int64_t *__restrict__ ids, int64_t n, int64
     const int64_t r = i / vocab, c = i - r * vocab;
     out[i] = (ids[r] == c) ? 1.0f : 0.0f;
   }
+}
+
+// draft [batch, k] as [k, batch]: the verdict's copy of the drafted ids, for the
+// kernels that do not write it
+__global__ void draft_rows_kernel(const int64_t *__restrict__ draft, int64_t batch, int64_t k,
+                                  int64_t *__restrict__ out) {
+  const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (i < batch * k) out[i % k * batch + i / k] = draft[i];
 }
 
 }  // namespace specdec
@@ -1387,12 +1403,12 @@ SPECDEC_API int specdec_accept_workspace(int64_t batch, int64_t *bytes) {
   return SPECDEC_OK;
 }
 
-SPECDEC_API int specdec_accept_reject(const void *p, const void *q, int dtype,
+static int accept_reject_call(const void *p, const void *q, int dtype,
                                       int64_t p_batch_stride, int64_t p_row_stride,
                                       int64_t q_batch_stride, int64_t q_row_stride,
                                       const int64_t *draft, const void *u_accept,
                                       const void *u_residual, int64_t batch, int64_t k,
-                                      int64_t vocab, int64_t *out, void *workspace,
+                                      int64_t vocab, int64_t *out, int64_t *draft_out, void *workspace,
                                       int64_t workspace_bytes, int32_t spin, void *stream) {
   if (batch < 0 || k < 0 || vocab <= 0) return SPECDEC_EINVAL;
   if (vocab > (int64_t)kMaxTiles * kCdfPerThread * kAcceptThreads) return SPECDEC_EUNSUPPORTED;
@@ -1414,6 +1430,7 @@ SPECDEC_API int specdec_accept_reject(const void *p, const void *q, int dtype,
     a.temperature = 1.0f;
     a.spin = spin;
     a.out = out;
+    a.draft_out = draft_out;
     a.ws = (uint64_t *)workspace;
     const bool vec4 = mw_vec4(p, q, p_batch_stride, p_row_stride, q_batch_stride, q_row_stride, k, vocab);
     switch (pl.E) {
@@ -1448,15 +1465,37 @@ SPECDEC_API int specdec_accept_reject(const void *p, const void *q, int dtype,
   } else {
     return SPECDEC_EINVAL;
   }
+  if (draft_out && k > 0)
+    draft_rows_kernel<<<(unsigned)((batch * k + 255) / 256), 256, 0, s>>>(draft, batch, k, draft_out);
   return launch_status();
 }
 
-SPECDEC_API int specdec_accept_reject_logits(const void *target_logits, const void *draft_logits, int dtype,
+SPECDEC_API int specdec_accept_reject(const void *p, const void *q, int dtype, int64_t p_batch_stride,
+                                      int64_t p_row_stride, int64_t q_batch_stride, int64_t q_row_stride,
+                                      const int64_t *draft, const void *u_accept, const void *u_residual,
+                                      int64_t batch, int64_t k, int64_t vocab, int64_t *out, void *workspace,
+                                      int64_t workspace_bytes, int32_t spin, void *stream) {
+  return accept_reject_call(p, q, dtype, p_batch_stride, p_row_stride, q_batch_stride, q_row_stride, draft, u_accept,
+                            u_residual, batch, k, vocab, out, nullptr, workspace, workspace_bytes, spin, stream);
+}
+
+SPECDEC_API int specdec_accept_verdict(const void *p, const void *q, int dtype, int64_t p_batch_stride,
+                                       int64_t p_row_stride, int64_t q_batch_stride, int64_t q_row_stride,
+                                       const int64_t *draft, const void *u_accept, const void *u_residual,
+                                       int64_t batch, int64_t k, int64_t vocab, int64_t *out, void *workspace,
+                                       int64_t workspace_bytes, int32_t spin, void *stream) {
+  return accept_reject_call(p, q, dtype, p_batch_stride, p_row_stride, q_batch_stride, q_row_stride, draft, u_accept,
+                            u_residual, batch, k, vocab, out, out ? out + 3 * batch : nullptr, workspace,
+                            workspace_bytes, spin, stream);
+}
+
+
+static int accept_logits_call(const void *target_logits, const void *draft_logits, int dtype,
                                              int64_t t_batch_stride, int64_t t_row_stride,
                                              int64_t d_batch_stride, int64_t d_row_stride, float temperature,
                                              const int64_t *draft, const void *u_accept,
                                              const void *u_residual, int64_t batch, int64_t k, int64_t vocab,
-                                             int64_t *out, void *workspace, int64_t workspace_bytes,
+                                             int64_t *out, int64_t *draft_out, void *workspace, int64_t workspace_bytes,
                                              int32_t spin, void *stream) {
   if (batch < 0 || k < 0 || vocab <= 0 || !(temperature >= 0.0f)) return SPECDEC_EINVAL;
   if (batch == 0) return SPECDEC_OK;
@@ -1482,6 +1521,7 @@ SPECDEC_API int specdec_accept_reject_logits(const void *target_logits, const vo
   a.temperature = temperature;
   a.spin = spin;
   a.out = out;
+  a.draft_out = draft_out;
   a.ws = (uint64_t *)workspace;
   hipStream_t s = as_stream(stream);
   switch (pl.E) {
@@ -1491,6 +1531,28 @@ SPECDEC_API int specdec_accept_reject_logits(const void *target_logits, const vo
     default: launch_mw_e<24, true>(true, a, s); break;
   }
   return launch_status();
+}
+
+SPECDEC_API int specdec_accept_reject_logits(const void *target_logits, const void *draft_logits, int dtype,
+                                             int64_t t_batch_stride, int64_t t_row_stride, int64_t d_batch_stride,
+                                             int64_t d_row_stride, float temperature, const int64_t *draft,
+                                             const void *u_accept, const void *u_residual, int64_t batch, int64_t k,
+                                             int64_t vocab, int64_t *out, void *workspace, int64_t workspace_bytes,
+                                             int32_t spin, void *stream) {
+  return accept_logits_call(target_logits, draft_logits, dtype, t_batch_stride, t_row_stride, d_batch_stride,
+                            d_row_stride, temperature, draft, u_accept, u_residual, batch, k, vocab, out, nullptr,
+                            workspace, workspace_bytes, spin, stream);
+}
+
+SPECDEC_API int specdec_accept_verdict_logits(const void *target_logits, const void *draft_logits, int dtype,
+                                              int64_t t_batch_stride, int64_t t_row_stride, int64_t d_batch_stride,
+                                              int64_t d_row_stride, float temperature, const int64_t *draft,
+                                              const void *u_accept, const void *u_residual, int64_t batch, int64_t k,
+                                              int64_t vocab, int64_t *out, void *workspace, int64_t workspace_bytes,
+                                              int32_t spin, void *stream) {
+  return accept_logits_call(target_logits, draft_logits, dtype, t_batch_stride, t_row_stride, d_batch_stride,
+                            d_row_stride, temperature, draft, u_accept, u_residual, batch, k, vocab, out,
+                            out ? out + 3 * batch : nullptr, workspace, workspace_bytes, spin, stream);
 }
 
 SPECDEC_API int specdec_accept_count(const void *p, const void *q, int dtype,

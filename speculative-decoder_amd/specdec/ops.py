@@ -73,7 +73,15 @@ def _token_rows(t: torch.Tensor, tokens: int, stride: int, row: int, name: str) 
                          f"elements at stride {stride} need {need}")
 
 
+# the current stream's handle without building a torch Stream around it (2.9 us
+# of a small call's 11 to 20 us on the host)
+_raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None)
+_device_index = getattr(torch._C, "_cuda_getDevice", None)
+
+
 def stream() -> int:
+    if _raw_stream is not None and _device_index is not None:
+        return _raw_stream(_device_index())
     return torch.cuda.current_stream().cuda_stream
 
 
@@ -170,34 +178,36 @@ ACCEPT_SPIN = 1 << 14
 
 
 def accept_reject(p, q, draft, u_accept, u_residual, workspace: AcceptWorkspace | None = None,
-                  single: bool = False, spin: int = ACCEPT_SPIN) -> torch.Tensor:
+                  single: bool = False, spin: int = ACCEPT_SPIN, with_draft: bool = False) -> torch.Tensor:
     """Fused accept + residual + inverse CDF; returns int64 [3, B] on the GPU:
     n_accepted, next_token, and a flag that is 1 for a drafted token with
     zero q(x) or outside the vocabulary.  `single` asks for the
     one-workgroup-per-row kernel (no workspace); `spin` bounds the waits of
     the many-CU kernel (negative: none; every workgroup then computes the
-    other chunks' values itself, with the same bits)."""
+    other chunks' values itself, with the same bits).  `with_draft` appends the
+    drafted ids, transposed: int64 [3 + k, B], for one copy to the host."""
     p, q = _rows3(gpu(p, "p")), _rows3(gpu(q, "q"))
     b, k = _accept_inputs(p, q, draft, u_accept)
     _on(p.device, u_residual, "u_residual", p.dtype, True, b)
-    out = torch.empty(3, b, dtype=torch.int64, device=p.device)
+    out = torch.empty(3 + k if with_draft else 3, b, dtype=torch.int64, device=p.device)
     ws_ptr, ws_bytes = None, 0
     if not single:
         buf = (workspace or accept_workspace_for(p.device)).reserve(b)
         ws_ptr, ws_bytes = buf.data_ptr(), buf.numel()
-    st = lib().specdec_accept_reject(p.data_ptr(), q.data_ptr(), dtype_code(p), p.stride(0), p.stride(1),
-                                     q.stride(0), q.stride(1), draft.data_ptr(), u_accept.data_ptr(),
-                                     u_residual.data_ptr(), b, k, p.shape[-1], out.data_ptr(), ws_ptr, ws_bytes,
-                                     int(spin), stream())
+    entry = lib().specdec_accept_verdict if with_draft else lib().specdec_accept_reject
+    st = entry(p.data_ptr(), q.data_ptr(), dtype_code(p), p.stride(0), p.stride(1), q.stride(0), q.stride(1),
+               draft.data_ptr(), u_accept.data_ptr(), u_residual.data_ptr(), b, k, p.shape[-1], out.data_ptr(), ws_ptr,
+               ws_bytes, int(spin), stream())
     _check(st, "accept_reject")
     return out
 
 
 def accept_reject_logits(target_logits, draft_logits, temperature: float, draft, u_accept, u_residual,
-                         workspace: AcceptWorkspace | None = None, spin: int = ACCEPT_SPIN) -> torch.Tensor | None:
+                         workspace: AcceptWorkspace | None = None, spin: int = ACCEPT_SPIN,
+                         with_draft: bool = False) -> torch.Tensor | None:
     """probabilities() of the target [B, k+1, V] and draft [B, k, V] fp32
     logits followed by accept_reject, in one launch that reads the logits
-    once; int64 [3, B] as accept_reject returns, or None when the shapes do
+    once; int64 [3, B] ([3 + k, B]) as accept_reject returns, or None when the shapes do
     not fit the kernel (more than 16 drafted positions, rows that are not
     16-byte aligned, too many rows for the GPU)."""
     tl, dl = _rows3(gpu(target_logits, "target_logits")), _rows3(gpu(draft_logits, "draft_logits"))
@@ -207,12 +217,12 @@ def accept_reject_logits(target_logits, draft_logits, temperature: float, draft,
     _on(tl.device, u_residual, "u_residual", tl.dtype, True, b)
     if temperature < 0:
         raise ValueError(f"temperature must be >= 0 (got {temperature})")
-    out = torch.empty(3, b, dtype=torch.int64, device=tl.device)
+    out = torch.empty(3 + k if with_draft else 3, b, dtype=torch.int64, device=tl.device)
     buf = (workspace or accept_workspace_for(tl.device)).reserve(b)
-    st = lib().specdec_accept_reject_logits(tl.data_ptr(), dl.data_ptr(), dtype_code(tl), tl.stride(0), tl.stride(1),
-                                            dl.stride(0), dl.stride(1), float(temperature), draft.data_ptr(),
-                                            u_accept.data_ptr(), u_residual.data_ptr(), b, k, tl.shape[-1],
-                                            out.data_ptr(), buf.data_ptr(), buf.numel(), int(spin), stream())
+    entry = lib().specdec_accept_verdict_logits if with_draft else lib().specdec_accept_reject_logits
+    st = entry(tl.data_ptr(), dl.data_ptr(), dtype_code(tl), tl.stride(0), tl.stride(1), dl.stride(0), dl.stride(1),
+               float(temperature), draft.data_ptr(), u_accept.data_ptr(), u_residual.data_ptr(), b, k, tl.shape[-1],
+               out.data_ptr(), buf.data_ptr(), buf.numel(), int(spin), stream())
     if st == EUNSUPPORTED:
         return None
     _check(st, "accept_reject_logits")

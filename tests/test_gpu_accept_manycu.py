@@ -137,3 +137,22 @@ def test_graph_replays_match_eager():
         torch.cuda.synchronize()
         assert torch.equal(out, want), i
         assert torch.equal(ops.accept_reject(p, q, draft, ua, ur, workspace=ws), want), i
+
+
+@pytest.mark.parametrize("b,k,v,dtype,single", [(1, 4, 49152, torch.float32, False), (5, 1, 1000, torch.float32, True),
+                                                (3, 300, 64, torch.float32, False), (4, 3, 97, torch.float64, False),
+                                                (2, 0, 512, torch.float32, False), (8, 8, 4096, torch.float32, False)])
+def test_the_draft_rides_behind_the_verdict(b, k, v, dtype, single):
+    """with_draft appends the drafted ids, transposed, to the same verdict (every kernel of the call)."""
+    g = torch.Generator().manual_seed(b + v)
+    p = torch.softmax(torch.randn(b, k + 1, v, generator=g), -1).to(dtype).cuda()
+    q = torch.softmax(torch.randn(b, k, v, generator=g), -1).to(dtype).cuda()
+    draft = torch.randint(0, v, (b, k), generator=g).cuda()
+    ua, ur = torch.rand(b, k, generator=g).to(dtype).cuda(), torch.rand(b, generator=g).to(dtype).cuda()
+    out = ops.accept_reject(p, q, draft, ua, ur, single=single, with_draft=True)
+    assert torch.equal(out[:3], ops.accept_reject(p, q, draft, ua, ur, single=single))
+    assert torch.equal(out[3:], draft.t())
+    if dtype == torch.float32 and k <= 16 and v % 4 == 0:
+        lg = ops.accept_reject_logits(p, q, 1.0, draft, ua, ur, with_draft=True)
+        assert torch.equal(lg[:3], ops.accept_reject_logits(p, q, 1.0, draft, ua, ur))
+        assert torch.equal(lg[3:], draft.t())
