@@ -1791,8 +1791,18 @@ attention_f32_groups_kernel(AttnArgs a) {
       }
     }
   };
-  auto compute = [&](const Chunk &x, int cs) {
+  auto compute = [&](Chunk &x, int cs) {
     if (cs >= s_hi) return;
+    if (cs + 32 > ti.kv_len) {  // slots past the keys: a weight of zero times what they hold
+#pragma unroll
+      for (int gi = 0; gi < 2; ++gi)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          const bool in = cs + 16 * gi + 4 * g + i < ti.kv_len;
+#pragma unroll
+          for (int j = 0; j < 4; ++j) x.v[gi][j][i] = in ? x.v[gi][j][i] : 0.0f;
+        }
+    }
     float sv[8];
 #pragma unroll
     for (int gi = 0; gi < 2; ++gi) {

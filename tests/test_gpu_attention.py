@@ -909,3 +909,43 @@ def test_latency_split_follows_the_keys_and_matches_the_default(batch, length, w
         outs.append(out.float())
     # a bf16 step of values below 1, and the weights' rounding to bf16
     assert (outs[0] - outs[1]).abs().max().item() < 1e-2
+
+
+@pytest.mark.parametrize("dtype,bs,total,t_new", [(torch.float32, 16, [21, 48, 70, 513], 5),
+                                                  (torch.float32, 32, [9, 33, 256, 530], 5),
+                                                  (torch.bfloat16, 16, [16, 48, 272, 528], 5),
+                                                  (torch.bfloat16, 32, [32, 64, 160, 544], 5),
+                                                  (torch.bfloat16, 16, [16, 528, 1040, 2064], 1)])
+def test_slots_past_the_keys_may_hold_anything(dtype, bs, total, t_new):
+    """A pool of NaN but for each row's history (blocks of freed sequences hold
+    whatever those left): the fused append's rows equal the oracle's.  bf16
+    rows end at a block's end, as its kernels read whole blocks."""
+    h, hkv, d = 4, 2, 64
+    g = torch.Generator().manual_seed(bs)
+    n = len(total)
+    cache = make_cache(1, hkv, d, sum(t // bs + 2 for t in total), bs, dtype, bs)
+    cache.k.fill_(float("nan"))
+    cache.v.fill_(float("nan"))
+    past = [t - t_new for t in total]
+    for s in range(n):
+        cache.add(s)
+    k, v = (torch.randn(n, hkv, max(total), d, generator=g).to(dtype) for _ in range(2))
+    step = cache.append(list(range(n)), past)
+    cache.write(0, step, k[:, :, :max(past)].cuda(), v[:, :, :max(past)].cuda())
+    step = cache.append(list(range(n)), [t_new] * n)
+    q = torch.randn(n, t_new, h, d, generator=g).to(dtype)
+    qkv = torch.empty(n, t_new, (h + 2 * hkv) * d, dtype=dtype)
+    for b in range(n):
+        new = slice(past[b], total[b])
+        qkv[b] = torch.cat([q[b].flatten(1), k[b, :, new].transpose(0, 1).flatten(1),
+                            v[b, :, new].transpose(0, 1).flatten(1)], dim=1)
+    cos, sin = torch.ones(max(total), d // 2, device="cuda"), torch.zeros(max(total), d // 2, device="cuda")
+    want = of.attention(q.transpose(1, 2).float(), k.float(), v.float(), torch.tensor(past), torch.tensor(total),
+                        0.125)
+    for split in (0, -1, 256):
+        out = torch.zeros(n, t_new, h * d, dtype=dtype, device="cuda")
+        ops.rope_paged_attention(qkv.cuda(), cos, sin, cache.k[0], cache.v[0], cache.table_tensor, step.meta, n, t_new,
+                                 h, hkv, d, bs, 0.125, max(total), out, out.stride(1), split_tokens=split)
+        got = out.view(n, t_new, h, d).transpose(1, 2).float().cpu()
+        # fp32 sums; bf16 outputs of magnitude up to 2, p rounded to bf16
+        assert (got - want).abs().max().item() < (2e-5 if dtype == torch.float32 else 2e-2), split
