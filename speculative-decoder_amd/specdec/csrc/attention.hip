@@ -626,14 +626,19 @@ attention_bf16_kernel(
     qraw[0] = *reinterpret_cast<const u32x4 *>(qr);
     qraw[1] = *reinterpret_cast<const u32x4 *>(qr + 32);
   }
-  const bool pre_norm = NW == 16 && MODE != 0 && a.hidden && a.hdim <= 4 * kWave * 8;
-  const int pre_tok = tid0 >> 6;
-  u32x4 hv_pre[4];
-  if (pre_norm && pre_tok < min(a.width, kStage)) {
+  constexpr int kPreRows = NW == 16 ? 1 : 2;  // residual rows a wave loads early: tokens w, w + NW
+  const bool pre_norm = MODE != 0 && a.hidden && a.hdim <= 4 * kWave * 8;
+  u32x4 hv_pre[kPreRows][4];
+  if (pre_norm && (NW != 16 || (tid0 >> 6) < a.width)) {
     const int nvec = a.hdim / 8;
-    const u32x4 *hr = reinterpret_cast<const u32x4 *>(a.hidden) + ((int64_t)ti.b * a.width + pre_tok) * nvec;
 #pragma unroll
-    for (int k = 0; k < 4; ++k) hv_pre[k] = hr[min(lane0 + kWave * k, nvec - 1)];
+    for (int i = 0; i < kPreRows; ++i) {
+      // (a token past the call's: the last one again, not used)
+      const int tok = min((tid0 >> 6) + NW * i, a.width - 1);
+      const u32x4 *hr = reinterpret_cast<const u32x4 *>(a.hidden) + ((int64_t)ti.b * a.width + tok) * nvec;
+#pragma unroll
+      for (int k = 0; k < 4; ++k) hv_pre[i][k] = hr[min(lane0 + kWave * k, nvec - 1)];
+    }
   }
   const bool pre_kv = NW == 16 && MODE != 0 && a.rope && a.width <= kStage;
   u16 sk1[kKT], sk2[kKT], svv[kVT];
@@ -752,6 +757,70 @@ attention_bf16_kernel(
     }
   }
 
+  // element offset of the (block, head) tile holding token pos
+  auto tile_of = [&](int pos) -> int64_t { return ((int64_t)trow[pos / bs] * Hkv + ti.h) * tile_elems; };
+  // K/V operands of one 64-token step
+  struct StepRegs {
+    u32x4 k[2][2][2];  // [chunk][half][kk]
+    u32x4 v[2][4];     // [chunk][dim tile]
+  };
+  // this lane's block ids for the step at c0 (lane j & 3: tokens c0 + 16j ..)
+  auto step_blocks = [&](int c0) -> int { return trow[min((c0 + 16 * (lane & 3)) / bs, last_blk)]; };
+  // Issue every K/V load of the step at c0; bjv holds its block ids.  Without
+  // conditions for whole 16-token groups, which kept the loads from going out
+  // together: a group past the keys reads the row's last block (its scores are
+  // masked and its V zeroed below), a slot that this call appends reads
+  // whatever the pool holds (replaced from LDS before it is used).
+  auto issue = [&](int c0, int bjv, StepRegs &r) {
+    // tile offsets of the step's four 16-token groups (MODE != 0), uniform
+    // across the wave; a lane picks between two of them with a select (a
+    // dynamically indexed array would be placed in memory)
+    int64_t tofs0 = 0, tofs1 = 0, tofs2 = 0, tofs3 = 0;
+    if (MODE != 0) {
+      tofs0 = ((int64_t)__builtin_amdgcn_readlane(bjv, 0) * Hkv + ti.h) * tile_elems;
+      tofs1 = ((int64_t)__builtin_amdgcn_readlane(bjv, 1) * Hkv + ti.h) * tile_elems;
+      tofs2 = ((int64_t)__builtin_amdgcn_readlane(bjv, 2) * Hkv + ti.h) * tile_elems;
+      tofs3 = ((int64_t)__builtin_amdgcn_readlane(bjv, 3) * Hkv + ti.h) * tile_elems;
+    }
+    auto group_tile = [&](int ch, bool upper) -> int64_t {
+      return ch == 0 ? (upper ? tofs1 : tofs0) : (upper ? tofs3 : tofs2);
+    };
+#pragma unroll
+    for (int ch = 0; ch < 2; ++ch) {
+      const int cs = c0 + 32 * ch;
+#pragma unroll
+      for (int hf = 0; hf < 2; ++hf) {
+        const int tok = cs + 8 * (c >> 2) + 4 * hf + (c & 3);
+        if (MODE == 0) r.k[ch][hf][0] = r.k[ch][hf][1] = u32x4{0u, 0u, 0u, 0u};
+        if (MODE != 0 || tok < kv_len) {
+          const int64_t to = (MODE != 0) ? group_tile(ch, (c >> 3) != 0) : tile_of(tok);
+          const u16 *kb = kp + to + (int64_t)(tok % bs) * kD + 8 * g;
+          r.k[ch][hf][0] = *reinterpret_cast<const u32x4 *>(kb);
+          r.k[ch][hf][1] = *reinterpret_cast<const u32x4 *>(kb + 32);
+        }
+      }
+      const int vt = cs + 8 * g;  // first of this lane group's 8 tokens
+      if (MODE != 0) {
+        const u16 *vb = vp + group_tile(ch, (g >> 1) != 0) + vt % bs;
+#pragma unroll
+        for (int tt = 0; tt < 4; ++tt)
+          r.v[ch][tt] = *reinterpret_cast<const u32x4 *>(vb + (int64_t)(16 * tt + c) * bs);
+      } else {
+        unsigned int w[4][4] = {};
+#pragma unroll
+        for (int i = 0; i < 8; ++i) {
+          const int pos = vt + i;
+          if (pos >= kv_len) continue;
+          const u16 *vb = vp + tile_of(pos) + pos % bs;
+#pragma unroll
+          for (int tt = 0; tt < 4; ++tt)
+            w[tt][i >> 1] |= (unsigned)vb[(int64_t)(16 * tt + c) * bs] << (16 * (i & 1));
+        }
+#pragma unroll
+        for (int tt = 0; tt < 4; ++tt) r.v[ch][tt] = u32x4{w[tt][0], w[tt][1], w[tt][2], w[tt][3]};
+      }
+    }
+  };
   // Q operand: lane (query c, group g) holds dims 8g..8g+7 (kk = 0) and
   // 32+8g..32+8g+7 (kk = 1) -- the two halves of 8 RoPE pairs
   // (loaded above for the call's rows; zeros for rows past the row's new
@@ -784,14 +853,34 @@ attention_bf16_kernel(
   if (norm_in) {
     const int nvec = a.hdim / 8;
     const int ntok = min(min(ti.nnew, a.width), kStage);
-    for (int tk = tid >> 6; tk < ntok; tk += NW) {
+    if (pre_norm) {
+#pragma unroll
+      for (int i = 0; i < kPreRows; ++i) {
+        const int tk = (tid >> 6) + NW * i;
+        if (tk >= ntok) break;
+        float ss = 0.0f;
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+          const bool in = lane + kWave * k < nvec;
+#pragma unroll
+          for (int e = 0; e < 8; ++e) {
+            const unsigned w = hv_pre[i][k][e >> 1];
+            const float x = __uint_as_float((e & 1) ? (w & 0xFFFF0000u) : (w << 16));
+            ss += in ? x * x : 0.0f;
+          }
+        }
+        ss = wave_sum_dpp(ss);
+        if (lane == 0) s_tok[tk] = rsqrtf(ss / (float)a.hdim + a.eps);
+      }
+    }
+    for (int tk = (tid >> 6) + (pre_norm ? NW * kPreRows : 0); tk < ntok; tk += NW) {
       const u32x4 *hr = reinterpret_cast<const u32x4 *>(a.hidden) + ((int64_t)ti.b * a.width + tk) * nvec;
       float ss = 0.0f;
       for (int base = 0; base < nvec; base += 4 * kWave) {
         u32x4 hv[4];
 #pragma unroll
         for (int k = 0; k < 4; ++k)
-          hv[k] = (pre_norm && base == 0) ? hv_pre[k] : hr[min(base + lane + kWave * k, nvec - 1)];
+          hv[k] = hr[min(base + lane + kWave * k, nvec - 1)];
 #pragma unroll
         for (int k = 0; k < 4; ++k) {
           const bool in = base + lane + kWave * k < nvec;
@@ -873,77 +962,11 @@ attention_bf16_kernel(
     __syncthreads();
   }
 
-  // element offset of the (block, head) tile holding token pos
-  auto tile_of = [&](int pos) -> int64_t { return ((int64_t)trow[pos / bs] * Hkv + ti.h) * tile_elems; };
   f32x4 o[4];
 #pragma unroll
   for (int tt = 0; tt < 4; ++tt) o[tt] = f32x4{0.f, 0.f, 0.f, 0.f};
   float m = -INFINITY, l = 0.0f;
 
-  // K/V operands of one 64-token step
-  struct StepRegs {
-    u32x4 k[2][2][2];  // [chunk][half][kk]
-    u32x4 v[2][4];     // [chunk][dim tile]
-  };
-  // this lane's block ids for the step at c0 (lane j & 3: tokens c0 + 16j ..)
-  auto step_blocks = [&](int c0) -> int { return trow[min((c0 + 16 * (lane & 3)) / bs, last_blk)]; };
-  // issue every K/V load of the step at c0; bjv holds its block ids
-  auto issue = [&](int c0, int bjv, StepRegs &r) {
-    // tile offsets of the step's four 16-token groups (MODE != 0), uniform
-    // across the wave; a lane picks between two of them with a select (a
-    // dynamically indexed array would be placed in memory)
-    int64_t tofs0 = 0, tofs1 = 0, tofs2 = 0, tofs3 = 0;
-    if (MODE != 0) {
-      tofs0 = ((int64_t)__builtin_amdgcn_readlane(bjv, 0) * Hkv + ti.h) * tile_elems;
-      tofs1 = ((int64_t)__builtin_amdgcn_readlane(bjv, 1) * Hkv + ti.h) * tile_elems;
-      tofs2 = ((int64_t)__builtin_amdgcn_readlane(bjv, 2) * Hkv + ti.h) * tile_elems;
-      tofs3 = ((int64_t)__builtin_amdgcn_readlane(bjv, 3) * Hkv + ti.h) * tile_elems;
-    }
-    auto group_tile = [&](int ch, bool upper) -> int64_t {
-      return ch == 0 ? (upper ? tofs1 : tofs0) : (upper ? tofs3 : tofs2);
-    };
-#pragma unroll
-    for (int ch = 0; ch < 2; ++ch) {
-      const int cs = c0 + 32 * ch;
-#pragma unroll
-      for (int hf = 0; hf < 2; ++hf) {
-        const int tok = cs + 8 * (c >> 2) + 4 * hf + (c & 3);
-        const bool ok = (MODE == 0) ? tok < kv_len : (tok / bs) * bs < kv_len;
-        const bool fresh = staged && tok >= p0 && tok < p1;  // appended by this call: from LDS
-        r.k[ch][hf][0] = r.k[ch][hf][1] = u32x4{0u, 0u, 0u, 0u};
-        if (ok && !fresh) {
-          const int64_t to = (MODE != 0) ? group_tile(ch, (c >> 3) != 0) : tile_of(tok);
-          const u16 *kb = kp + to + (int64_t)(tok % bs) * kD + 8 * g;
-          r.k[ch][hf][0] = *reinterpret_cast<const u32x4 *>(kb);
-          r.k[ch][hf][1] = *reinterpret_cast<const u32x4 *>(kb + 32);
-        }
-      }
-      const int vt = cs + 8 * g;  // first of this lane group's 8 tokens
-#pragma unroll
-      for (int tt = 0; tt < 4; ++tt) r.v[ch][tt] = u32x4{0u, 0u, 0u, 0u};
-      if (MODE != 0) {
-        if ((vt / bs) * bs < kv_len) {
-          const u16 *vb = vp + group_tile(ch, (g >> 1) != 0) + vt % bs;
-#pragma unroll
-          for (int tt = 0; tt < 4; ++tt)
-            r.v[ch][tt] = *reinterpret_cast<const u32x4 *>(vb + (int64_t)(16 * tt + c) * bs);
-        }
-      } else {
-        unsigned int w[4][4] = {};
-#pragma unroll
-        for (int i = 0; i < 8; ++i) {
-          const int pos = vt + i;
-          if (pos >= kv_len) continue;
-          const u16 *vb = vp + tile_of(pos) + pos % bs;
-#pragma unroll
-          for (int tt = 0; tt < 4; ++tt)
-            w[tt][i >> 1] |= (unsigned)vb[(int64_t)(16 * tt + c) * bs] << (16 * (i & 1));
-        }
-#pragma unroll
-        for (int tt = 0; tt < 4; ++tt) r.v[ch][tt] = u32x4{w[tt][0], w[tt][1], w[tt][2], w[tt][3]};
-      }
-    }
-  };
   // keys appended by this call: K rows and V elements from LDS, then the
   // step's scores, online softmax and P V
   auto compute = [&](int c0, StepRegs &r) {
@@ -991,12 +1014,17 @@ attention_bf16_kernel(
     // reaching beyond `past`; elsewhere every score is visible
     if (c0 + 64 > ti.past) {
 #pragma unroll
-      for (int ch = 0; ch < 2; ++ch)
+      for (int ch = 0; ch < 2; ++ch) {
 #pragma unroll
         for (int j = 0; j < 8; ++j) {
           const int pos = c0 + 32 * ch + 8 * g + j;
           if (!(row_ok && pos <= qpos && pos < kv_len)) sv[8 * ch + j] = -INFINITY;
         }
+        // (a weight of zero times what a slot past the keys holds)
+        const bool live = c0 + 32 * ch + 8 * g < kv_len;
+#pragma unroll
+        for (int tt = 0; tt < 4; ++tt) r.v[ch][tt] = live ? r.v[ch][tt] : u32x4{0u, 0u, 0u, 0u};
+      }
     }
     online_update<16>(sv, m, l, o);
 #pragma unroll
