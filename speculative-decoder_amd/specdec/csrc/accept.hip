@@ -732,7 +732,9 @@ __device__ __forceinline__ void mw_advance(uint64_t *ws, uint64_t epoch, uint64_
 // pay[c * per + i]; miss[c] = 1 for a chunk with a word still missing after
 // the first read and `spin` more rounds (every word is missing for
 // spin < 0).  A thread reads up to kMwPoll words per pass, all issued
-// before any is checked; more words than kMwPoll * 256 take more passes.
+// before any is checked; more words than kMwPoll * 256 take more passes.  Each
+// wave reads on by itself until its words are there, so that one barrier ends
+// a pass (a barrier in every round added its skew to each round trip).
 // Returns whether any chunk is missing (the same in every thread); ends
 // with a barrier.
 constexpr int kMwPoll = 4;
@@ -741,7 +743,6 @@ __device__ bool gather_meeting(const uint64_t *slots, int G, int per, int own, u
   const int tid = threadIdx.x, n = G * per;
   bool late = false;
   for (int c = tid; c < G; c += kMwThreads) miss[c] = 0;
-  if (spin < 0) __syncthreads();  // otherwise the rounds' barriers order the zeroing before any mark
   for (int i0 = 0; i0 < n; i0 += kMwPoll * kMwThreads) {
     unsigned pending = 0;  // bit j: word i0 + tid + j * kMwThreads not seen yet
 #pragma unroll
@@ -749,29 +750,29 @@ __device__ bool gather_meeting(const uint64_t *slots, int G, int per, int own, u
       const int i = i0 + tid + j * kMwThreads;
       if (i < n && i / per != own) pending |= 1u << j;
     }
-    if (spin >= 0) {
-      for (int round = 0;; ++round) {
-        uint64_t w[kMwPoll];
+    for (int round = 0; round <= spin && __builtin_amdgcn_ballot_w64(pending != 0u); ++round) {
+      if (round > 0) __builtin_amdgcn_s_sleep(1);
+      uint64_t w[kMwPoll];
 #pragma unroll
-        for (int j = 0; j < kMwPoll; ++j)
-          w[j] = (pending >> j & 1u) ? get_word(slots + i0 + tid + j * kMwThreads) : 0;
+      for (int j = 0; j < kMwPoll; ++j)
+        w[j] = (pending >> j & 1u) ? get_word(slots + i0 + tid + j * kMwThreads) : 0;
 #pragma unroll
-        for (int j = 0; j < kMwPoll; ++j) {
-          if ((pending >> j & 1u) && (uint32_t)(w[j] >> 32) == tag) {
-            pay[i0 + tid + j * kMwThreads] = (uint32_t)w[j];
-            pending &= ~(1u << j);
-          }
+      for (int j = 0; j < kMwPoll; ++j) {
+        if ((pending >> j & 1u) && (uint32_t)(w[j] >> 32) == tag) {
+          pay[i0 + tid + j * kMwThreads] = (uint32_t)w[j];
+          pending &= ~(1u << j);
         }
-        if (!__syncthreads_or(pending != 0u) || round >= spin) break;
-        __builtin_amdgcn_s_sleep(1);
       }
     }
+    if (__syncthreads_or(pending != 0u)) {  // (also orders the zeroing of miss before any mark)
+      late = true;
 #pragma unroll
-    for (int j = 0; j < kMwPoll; ++j)
-      if (pending >> j & 1u) miss[(i0 + tid + j * kMwThreads) / per] = 1;
-    late |= pending != 0u;
+      for (int j = 0; j < kMwPoll; ++j)
+        if (pending >> j & 1u) miss[(i0 + tid + j * kMwThreads) / per] = 1;
+    }
   }
-  return __syncthreads_or(late);
+  if (late) __syncthreads();
+  return late;
 }
 
 // ---- statistics of the logits form (meeting A) ----
@@ -790,6 +791,30 @@ __device__ __forceinline__ const float *logit_row(const float *t_b, const float 
 // VGPRs: 72 or 48 elements in flight per thread (nine rows at E = 16 take
 // 256 VGPRs and 163 AGPRs).
 constexpr int mw_rows_per_batch(int E) { return E == 8 || E == 16 ? 9 : E == 12 ? 6 : E >= 48 ? 1 : 48 / E; }
+
+// x[e] /= T, correctly rounded (inv = 1 / T, correctly rounded).  With that
+// inv, one correction by the exact remainder of the product rounds as the
+// division does (Markstein 1990), unless the remainder leaves the normal
+// range: numbers of 1e18 and more and infinities, or an extreme T, take the
+// division itself, and quotients below 1e-18 may keep a rounding that no
+// difference of two logits shows.  The division's 14 or so operations on each
+// of 27 M logits were 7 of this kernel's 51 us (batch 32, k = 8); T is the
+// same for all of them.
+template <int E> __device__ __forceinline__ void divide_all(float (&x)[E], float T, float inv) {
+  float top = 0.0f;
+#pragma unroll
+  for (int e = 0; e < E; ++e) top = fmaxf(top, fabsf(x[e]));
+  if (__builtin_amdgcn_ballot_w64(!(top < 1e18f && T > 1e-18f && T < 1e18f))) {
+#pragma unroll
+    for (int e = 0; e < E; ++e) x[e] = x[e] / T;
+  } else {
+#pragma unroll
+    for (int e = 0; e < E; ++e) {
+      const float q = x[e] * inv;
+      x[e] = __builtin_fmaf(__builtin_fmaf(-T, q, x[e]), inv, q);
+    }
+  }
+}
 
 // Meeting A payloads of chunk gc, every logit row: pay[2r] = the max bits,
 // pay[2r + 1] = the sum bits (T > 0) or the index (T = 0).  RB rows are
@@ -812,6 +837,7 @@ __device__ __forceinline__ void chunk_stats(const float *t_b, const float *d_b, 
   constexpr int nw = kMwThreads / kWave;
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const unsigned first = (unsigned)gc * (kMwThreads * E) + (unsigned)tid * E;
+  const float inv = 1.0f / T;
   // every load unconditional (rows past R load row R - 1 again, unused):
   // a row filled with zeros on one path and loaded on another made the
   // compiler wait for each row's loads before the next row's went out
@@ -850,9 +876,7 @@ __device__ __forceinline__ void chunk_stats(const float *t_b, const float *d_b, 
     // y = l / T (x / 1 is x exactly: no division at T = 1); -inf past the row
     if (T != 1.0f) {
 #pragma unroll
-      for (int rb = 0; rb < RB; ++rb)
-#pragma unroll
-        for (int e = 0; e < E; ++e) v[rb][e] = v[rb][e] / T;
+      for (int rb = 0; rb < RB; ++rb) divide_all(v[rb], T, inv);
     }
     float mt[RB];
 #pragma unroll
@@ -1014,12 +1038,11 @@ __device__ __forceinline__ Chain chain_sum(const uint32_t *pay, int n, int j) {
 template <int E, bool VEC4, bool LOGITS>
 __global__ __launch_bounds__(kMwThreads) void accept_reject_mw_kernel(MwArgs a) {
   __shared__ double scratch[kMwThreads / kWave + 1];
-  __shared__ uint32_t s_pay[2 * kMwMaxR * kMwMaxG];  // one meeting's payloads
+  __shared__ __align__(8) uint32_t s_pay[2 * kMwMaxR * kMwMaxG];  // one meeting's payloads
   __shared__ int s_miss[kMwMaxG];
   __shared__ float s_fin[LOGITS ? kMwMaxR : 1][2];   // per logit row: (M, 1 / S) or (max, index)
-  __shared__ float s_terms[LOGITS ? kMwMaxR * kMwMaxG : 1];  // the fold's per-chunk terms
   __shared__ float s_red[LOGITS ? mw_rows_per_batch(E) : 1][4][2];
-  __shared__ int s_flag[LOGITS ? kMwMaxK : 1];        // bit 0: rejected, bit 1: bad draft
+  __shared__ int s_n[2];                             // logits form: n, the bad-draft flag
   __shared__ double s_last;
   const int G = a.G;
   const int64_t b = blockIdx.x / G, k = a.k, vocab = a.vocab;
@@ -1102,65 +1125,69 @@ __global__ __launch_bounds__(kMwThreads) void accept_reject_mw_kernel(MwArgs a) 
         if (s_miss[c])
           chunk_stats<E, VEC4>(t_b, d_b, a.p_rs, a.q_rs, k, vocab, a.temperature, c, R, pay + 2 * R * c, s_red,
                                [] {});
-    // every row's (M, 1 / S) -- or (max, index) -- folded over the chunks:
-    // M = the chunks' max (one wave per row, lane c holding chunk c: a max,
-    // or a (max, lowest index) merge, has the same result in any order);
-    // S = the sum over chunks, in chunk order, of S_c 2^((M_c - M) log2 e),
-    // the terms computed one per thread
-    {
-      const int lane = tid & (kWave - 1);
-      for (int r = tid / kWave; r < R; r += kMwThreads / kWave) {
-        float m = lane < G ? __uint_as_float(pay[2 * R * lane + 2 * r]) : -INFINITY;
-        int idx = lane < G ? (int)pay[2 * R * lane + 2 * r + 1] : INT32_MAX;
-        if (a.temperature == 0.0f) wave_argmax_dpp(m, idx);
-        else m = wave_max_dpp(m);
-        if (lane == 0) {
-          s_fin[r][0] = m;
-          s_fin[r][1] = __int_as_float(idx);
-        }
-      }
-    }
-    __syncthreads();
-    if (a.temperature != 0.0f) {
+    // every row's (M, 1 / S) -- or (max, index) -- folded over the chunks,
+    // and the accept test of every position, u * q(x) < p(x), by one wave
+    // without a barrier: lane r takes row r through the chunks (R <= 33) and
+    // lane t position t.  M = the chunks' max (a max, or a (max, lowest index)
+    // merge); S = the sum, in chunk order, of S_c 2^((M_c - M) log2 e).
+    // (The chain of meetings is what this kernel's time is beyond its reads:
+    // 18 us of 44 at batch 32, k = 8.  Terms spread over the workgroup's
+    // threads, with four barriers, took 2.9 us of it; this takes 1.7.)
+    if (tid < kWave) {
 #pragma clang fp contract(off)
-      for (int i = tid; i < R * G; i += kMwThreads) {
-        const int r = i / G, c = i - r * G;
-        const float mc = __uint_as_float(pay[2 * R * c + 2 * r]), sc = __uint_as_float(pay[2 * R * c + 2 * r + 1]);
-        s_terms[i] = mc == -INFINITY ? 0.0f : sc * __builtin_amdgcn_exp2f((mc - s_fin[r][0]) * kMwLog2e);
-      }
-      __syncthreads();
-      if (tid < R) {
+      const int r = min(tid, R - 1);
+      auto pair = [&](int c) { return *reinterpret_cast<const uint2 *>(&pay[2 * (R * c + r)]); };
+      float m = -INFINITY, second;
+      if (a.temperature == 0.0f) {
+        int idx = INT32_MAX;
+        for (int c = 0; c < G; ++c) {
+          const uint2 w = pair(c);
+          argmax_merge(m, idx, __uint_as_float(w.x), (int)w.y);
+        }
+        second = __int_as_float(idx);
+      } else {
+        for (int c0 = 0; c0 < G; c0 += 16)
+#pragma unroll
+          for (int i = 0; i < 16; ++i) m = fmaxf(m, __uint_as_float(pair(min(c0 + i, G - 1)).x));
         float sum = 0.0f;
-        for (int c0 = 0; c0 < G; c0 += 16) {  // each 16 terms read together, added in order
+        for (int c0 = 0; c0 < G; c0 += 16) {  // each 16 terms formed together, added in order
           float t[16];
 #pragma unroll
-          for (int i = 0; i < 16; ++i) t[i] = s_terms[tid * G + min(c0 + i, G - 1)];
+          for (int i = 0; i < 16; ++i) {
+            const uint2 w = pair(min(c0 + i, G - 1));
+            const float mc = __uint_as_float(w.x), sc = __uint_as_float(w.y);
+            t[i] = mc == -INFINITY || c0 + i >= G ? 0.0f : sc * __builtin_amdgcn_exp2f((mc - m) * kMwLog2e);
+          }
 #pragma unroll
-          for (int i = 0; i < 16; ++i)
-            if (c0 + i < G) sum += t[i];
+          for (int i = 0; i < 16; ++i) sum += t[i];  // (zeros past the chunks)
         }
-        s_fin[tid][1] = 1.0f / sum;
+        second = 1.0f / sum;
       }
-      __syncthreads();
-    }
-    // the accept test of every position: u * q(x) < p(x)
-    if (tid < k) {
-      int f = 0;
-      if (xid < 0 || xid >= vocab) {
-        f = 3;
-      } else {
-        const float px = prob_of(lt, xid, a.temperature, s_fin[tid][0], s_fin[tid][1]);
-        const float qx = prob_of(ld, xid, a.temperature, s_fin[k + 1 + tid][0], s_fin[k + 1 + tid][1]);
-        f = (uacc * qx < px ? 0 : 1) | (qx > 0.0f ? 0 : 2);
+      if (tid < R) {
+        s_fin[tid][0] = m;
+        s_fin[tid][1] = second;
       }
-      s_flag[tid] = f;
+      const float mq = __shfl(m, (int)k + 1 + tid, kWave), iq = __shfl(second, (int)k + 1 + tid, kWave);
+      bool rejected = false, wrong = false;
+      if (tid < k) {
+        if (xid < 0 || xid >= vocab) {
+          rejected = wrong = true;
+        } else {
+          const float px = prob_of(lt, xid, a.temperature, m, second);
+          const float qx = prob_of(ld, xid, a.temperature, mq, iq);
+          rejected = !(uacc * qx < px);
+          wrong = !(qx > 0.0f);
+        }
+      }
+      const uint64_t rej = __builtin_amdgcn_ballot_w64(rejected), any_bad = __builtin_amdgcn_ballot_w64(wrong);
+      if (tid == 0) {
+        s_n[0] = rej ? __builtin_ctzll(rej) : (int)k;
+        s_n[1] = any_bad != 0;
+      }
     }
     __syncthreads();
-    for (int64_t t = 0; t < k; ++t) {
-      const int f = s_flag[t];
-      if (f & 2) bad = 1;
-      if (n == k && (f & 1)) n = t;
-    }
+    n = __builtin_amdgcn_readfirstlane(s_n[0]);
+    bad = s_n[1];
   } else {
     // the accept count n and the bad-draft flag, the same in every thread
     // (accept_stage's test, u * q(x) < p(x) as a product; an id outside the
@@ -1361,7 +1388,8 @@ SPECDEC_API int specdec_probabilities(const void *logits, int dtype, int64_t row
 // compute unit (E = 8, then 16), beyond that two, with narrower loads
 // (E = 12, then 24: up to 64 rows on 256 compute units), so that a compute
 // unit's second workgroup loads while the first reduces (batch 32, k = 8:
-// 53.3 -> 44.6 us; batch 64: 85 -> 66 us).  Every workgroup of a grid is
+// 53.3 -> 44.6 us; batch 64: 85 -> 66 us; with
+// the cheaper division and meetings since, 40.6 and 64).  Every workgroup of a grid is
 // resident at once when the GPU is otherwise idle; when it is not, the
 // meetings' fallback finishes the call with the same bits.
 struct MwPlan {

@@ -249,3 +249,19 @@ def test_graph_replays_match_eager():
         torch.cuda.synchronize()
         assert torch.equal(out, want), i
         assert torch.equal(ops.accept_reject_logits(*args, workspace=ws), want), i
+
+
+@pytest.mark.parametrize("b", [1, 32])
+@pytest.mark.parametrize("scale", [1e-20, 1e-10, 1.0, 1e17, 1e22])
+def test_temperatures_and_logits_of_any_size(b, scale):
+    """l / T by the reciprocal and one correction, or by the division where
+    the logits or T leave its range (1e18 and more, infinities): scaling both
+    leaves the distribution, and masked tokens (-inf) take no part."""
+    k, v, temperature = 4, 40004, 0.7 * scale
+    tl, dl, g = logits(b, k, v, seed=b)
+    tl, dl = tl * scale, dl * scale
+    tl[..., 100:9000] = -torch.inf
+    dl[..., 100:9000] = -torch.inf
+    draft = drafts_from(dl, temperature, g)
+    ua, ur = torch.rand(b, k, generator=g), torch.rand(b, generator=g)
+    check_vs_oracle(tl, dl, temperature, draft, ua, ur, fused(tl, dl, temperature, draft, ua, ur))
