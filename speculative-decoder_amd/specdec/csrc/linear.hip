@@ -183,6 +183,115 @@ __global__ __launch_bounds__(kLinMaxWaves * 64) void linear_kernel(LinArgs a) {
   }
 }
 
+// At most 8 rows of a weight with fewer feature tiles than half the compute
+// units: a workgroup takes 8 features.  A wave's MFMAs multiply two of
+// linear_kernel's k-splits ("chains") at once, chain w in the operands' lanes
+// c < 8 (8 features, 8 rows) and chain w + waves in lanes c >= 8: the diagonal
+// blocks of D are the two chains' sums, the other two are not used.  Every lane
+// loads (a tile cut in two left half of each load's lanes empty, of W and of x),
+// so half the load instructions request the same bytes, and with KB = 16 a
+// wave has all of K <= 8192 in flight at once.  The chains are added in order:
+// the bits of linear_kernel.  1.7B down (33.5 MB), 1 / 5 / 8 rows: 8.6 / 9.5 /
+// 11.0 us, 4.3 to 3.5 TB/s with the launch (one workgroup a tile 11.2 / 12.7 /
+// 13.9, a tile in two with half the lanes empty 11.1 at 5 rows); what is left
+// beyond W's bytes is the launch and x, which every workgroup reads.
+template <int KB>
+__global__ __launch_bounds__(kLinMaxWaves / 2 * 64) void linear_pairs_kernel(LinArgs a, int nw) {
+  __shared__ f32x4 s_acc[kLinMaxWaves][16];  // [chain][8 (features / 4) + row]
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, waves = blockDim.x >> 6;
+  const int c = lane & 15, g = lane >> 4, r = c & 7;
+  const int tile = blockIdx.x >> 1, half = blockIdx.x & 1;
+  const int n0 = tile * 16 + 8 * half;
+  const int chain = wave + (c >> 3) * waves, s_lo = chain * a.per_wave;
+  const int cnt = chain < nw ? max(min(a.per_wave, a.steps - s_lo), 0) : 0;
+  const int most = max(min(a.per_wave, a.steps - wave * a.per_wave), 0);  // the first chain has no fewer
+  // W rows past N read the last row (never stored); x rows past M, and both
+  // operands past a chain's steps, read zeros
+  const __amdgpu_buffer_rsrc_t wb = __builtin_amdgcn_make_buffer_rsrc(
+      const_cast<uint16_t *>(a.w), 0, (int)((int64_t)a.N * a.w_stride * 2), 0x00020000);
+  const __amdgpu_buffer_rsrc_t xb = __builtin_amdgcn_make_buffer_rsrc(
+      const_cast<uint16_t *>(a.x), 0, (int)(((int64_t)(a.M - 1) * a.x_stride + a.K) * 2), 0x00020000);
+  unsigned wbase, wstep;
+  w_lane(a, tile, min(n0 + r, a.N - 1), (lane & 48) | (8 * half + r), wbase, wstep);
+  const unsigned xbase = (unsigned)(((int64_t)r * a.x_stride + 8 * g) * 2);
+  // the result: lane 8 f + row of wave 0, features n0 + 4f ..; accumulate's
+  // values loaded now, as in linear_kernel
+  const int f0 = n0 + 4 * ((lane >> 3) & 1);
+  uint16_t pre[4];
+  {
+    const int obytes = a.accumulate ? (int)(((int64_t)(a.M - 1) * a.out_stride + a.N) * 2) : 0;
+    const __amdgpu_buffer_rsrc_t ob = __builtin_amdgcn_make_buffer_rsrc(a.out, 0, obytes, 0x00020000);
+    const unsigned obase = (unsigned)(((int64_t)r * a.out_stride + f0) * 2);
+#pragma unroll
+    for (int i = 0; i < 4; ++i) pre[i] = __builtin_amdgcn_raw_buffer_load_b16(ob, obase + 2u * i, 0, 0);
+  }
+  f32x4 acc = f32x4{0.f, 0.f, 0.f, 0.f};
+  u32x4 A0[KB], A1[KB], B0[KB], B1[KB];
+  auto issue = [&](u32x4 (&A)[KB], u32x4 (&B)[KB], int b) {
+#pragma unroll
+    for (int j = 0; j < KB; ++j) {
+      const int t = b * KB + j;
+      const unsigned s = (unsigned)(s_lo + t);
+      A[j] = __builtin_amdgcn_raw_buffer_load_b128(wb, t < cnt ? wbase + s * wstep : 0xFFFFFF00u, 0, 0);
+      B[j] = __builtin_amdgcn_raw_buffer_load_b128(xb, t < cnt ? xbase + s * 64u : 0xFFFFFF00u, 0, 0);
+    }
+  };
+  auto consume = [&](const u32x4 (&A)[KB], const u32x4 (&B)[KB], int b) {
+#pragma unroll
+    for (int j = 0; j < KB; ++j)
+      if (b * KB + j < most)
+        acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, A[j]),
+                                                      __builtin_bit_cast(bf16x8, B[j]), acc, 0, 0, 0);
+  };
+  const int nb = (most + KB - 1) / KB;
+  if (nb > 0) {
+    issue(A0, B0, 0);
+    __builtin_amdgcn_sched_barrier(0);
+    int b = 0;
+    for (; b + 2 < nb; b += 2) {
+      issue(A1, B1, b + 1);
+      __builtin_amdgcn_sched_barrier(0);
+      consume(A0, B0, b);
+      __builtin_amdgcn_sched_barrier(0);
+      issue(A0, B0, b + 2);
+      __builtin_amdgcn_sched_barrier(0);
+      consume(A1, B1, b + 1);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+    if (b + 1 < nb) {
+      issue(A1, B1, b + 1);
+      __builtin_amdgcn_sched_barrier(0);
+      consume(A0, B0, b);
+      __builtin_amdgcn_sched_barrier(0);
+      consume(A1, B1, b + 1);
+    } else {
+      consume(A0, B0, b);
+    }
+  }
+  if ((g >> 1) == (c >> 3) && chain < nw) s_acc[chain][8 * (g & 1) + r] = acc;
+  __syncthreads();
+  if (wave == 0 && lane < 16 && r < a.M) {
+    f32x4 t = s_acc[0][lane];
+    for (int w = 1; w < nw; ++w) t += s_acc[w][lane];
+    uint16_t *dst = a.out + (int64_t)r * a.out_stride + f0;
+    uint16_t o[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      float v = t[i];
+      if (a.accumulate && f0 + i < a.N) v += bf16_bits_to_f32(pre[i]);
+      o[i] = __builtin_bit_cast(uint16_t, __float2bfloat16(v));  // round to nearest even
+    }
+    if (f0 + 3 < a.N && ((uintptr_t)dst & 7) == 0) {
+      *reinterpret_cast<u32x2 *>(dst) =
+          u32x2{(uint32_t)o[0] | ((uint32_t)o[1] << 16), (uint32_t)o[2] | ((uint32_t)o[3] << 16)};
+    } else {
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+        if (f0 + i < a.N) dst[i] = o[i];
+    }
+  }
+}
+
 // linear_kernel<KB> of the attention rows a draft decode step left as
 // split partials (attention_decode_parts_kernel: `nparts` per row and query
 // head): each workgroup first folds them into its LDS copy of the rows --
@@ -829,13 +938,19 @@ SPECDEC_API int specdec_linear(const void *x, int64_t x_stride, const void *w, i
   if (rows <= 16) {
     // From 9 rows x outweighs W's latency where every compute unit has a tile:
     // two tiles share x through LDS (1.7B qkv, 16 rows: 8.1 against 9.5 us; 5
-    // rows 7.7 against 7.6).  With less than half a tile for each, two
-    // workgroups take a tile's features (1.7B down, 5 rows: 11.1 against 12.7
-    // us, o 5.1 against 5.4, draft down 3.6 against 3.7); a short projection
-    // gains nothing once x weighs in (draft down, 9 rows: 4.1 against 3.9) or
-    // without the residual (draft qkv, 5 rows: 2.87 against 2.79).
+    // rows 7.7 against 7.6).  With less than half a tile for each, workgroups
+    // of 8 features fill the chip: linear_pairs_kernel up to 8 rows (5 rows,
+    // against a workgroup a tile: 1.7B down 9.5 and 12.7 us, o 4.3 and 5.4,
+    // draft down 3.3 and 3.8, draft qkv 2.78 and 2.82; with more tiles its
+    // launch is too many workgroups, 1.7B qkv 8.1 and 7.7), and above it, for
+    // a long projection only, a tile in two (draft down, 9 rows: 4.1 against
+    // 3.9).
     if (rows > 8 && tiles >= cus) launch_linear_rows<1, 2, 4>(a, tiles, waves, s);
-    else if (2 * tiles <= cus && (a.steps >= 64 || (a.accumulate && rows <= 8)))
+    else if (2 * tiles <= cus && rows <= 8) {
+      const dim3 pg((unsigned)(2 * tiles)), pb((unsigned)(64 * ((waves + 1) / 2)));
+      if (a.per_wave > 8) linear_pairs_kernel<16><<<pg, pb, 0, s>>>(a, waves);
+      else linear_pairs_kernel<8><<<pg, pb, 0, s>>>(a, waves);
+    } else if (2 * tiles <= cus && a.steps >= 64)
       linear_kernel<8, 2><<<dim3((unsigned)(2 * tiles)), block, 0, s>>>(a);
     else linear_kernel<8, 1><<<grid, block, 0, s>>>(a);
     return launch_status();

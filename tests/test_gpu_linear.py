@@ -186,12 +186,13 @@ def test_linear_silu_tiled_weight_gives_the_same_bits(rows, k, inter):
 # every instance of the kernels for more rows and its edges: column tiles to
 # workgroups of their own (few feature tiles), one workgroup of 3 or 4, two
 # feature tiles a workgroup with an odd count, a ragged k-split, a last chunk
-# of one k-step, rows one past a column tile
+# of one k-step, rows one past a column tile, k-splits of odd count and of
+# unequal length
 @pytest.mark.parametrize("rows,k,n,tiled", [(17, 576, 960, True), (33, 2048, 2048, True), (49, 96, 3088, True),
                                             (40, 160, 3000, False), (20, 96, 4112, True), (48, 288, 4112, True),
                                             (64, 2080, 4100, False), (41, 1056, 2208, True), (64, 32, 33, False),
                                             (16, 288, 4112, True), (9, 2048, 4100, False), (8, 576, 576, True),
-                                            (16, 2112, 2048, True)])
+                                            (16, 2112, 2048, True), (17, 8192, 40, False), (20, 2112, 112, True)])
 def test_more_rows_equal_few_at_a_time_bitwise(rows, k, n, tiled):
     x, w = operands(rows, k, n, seed=rows + n)
     xd, wd = x.to(DEV), w.to(DEV)
