@@ -822,9 +822,11 @@ def latency_split(batch: int, width: int, n_heads: int, n_kv_heads: int, max_kv_
     (32 rows at 2000: 18.6 against 17.7).  Past 2048 keys one workgroup per
     unit takes a microsecond for each 170 keys (one row of 4000: 25.6 us), so
     the keys are split: by 256 while that gives at most four workgroups per
-    compute unit (10.9 us), else by 512 (32 rows of 2500: 18.0 against 19.9)."""
+    compute unit (10.9 us), else by 512 (32 rows of 2500: 18.0 against 19.9).
+    Calls of several query tiles per unit (prompts) keep -1 or 0 at any length:
+    0's splits grow with their many units, which bounds their workspace."""
     units = batch * n_kv_heads * -(-(width * (n_heads // n_kv_heads)) // 16)
-    if max_kv_len <= 2048:
+    if max_kv_len <= 2048 or width * (n_heads // n_kv_heads) > 16:
         return -1 if units < 64 or width == 1 else 0
     return 256 if units * -(-max_kv_len // 256) <= 1024 else 512
 

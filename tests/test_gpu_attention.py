@@ -890,6 +890,8 @@ def test_latency_split_follows_the_keys_and_matches_the_default(batch, length, w
     max_kv = 2048 if length < 2048 else 4096
     split = ops.latency_split(batch, 1, h, hkv, max_kv)
     assert split == want
+    # a prompt's split, and with it its workspace, is the default's or none
+    assert ops.latency_split(1, 20, h, hkv, 4096) == -1 and ops.latency_split(batch, 3000, h, hkv, max_kv) == 0
     g = torch.Generator(device="cuda").manual_seed(batch)
     cache = KVCache(1, hkv, d, batch * (length // bs + 2), bs, torch.bfloat16, "cuda")
     ids = list(range(batch))
