@@ -6,7 +6,7 @@ A forward is split in two:
   * device part, `forward_core`: five launches per layer for decode,
     verification and draft steps (six when the attention needs its split
     combine):
-      - the fused QKV projection (specdec_linear at decode sizes, else
+      - the fused QKV projection (specdec_linear up to 64 rows, else
         torch/hipBLASLt) of the unnormalised residual stream;
       - the paged attention kernel, which finishes the input RMSNorm (each
         token's q/k/v scaled by its row's rsqrt(mean(x^2) + eps)), applies
@@ -197,7 +197,7 @@ def forward(model, cache: KVCache, seq_ids: list[int], input_ids: torch.Tensor, 
     speculative verification (T = k + 1).  `latency_split` lets attention
     pick a split for latency (the draft) instead of the fixed default.  With
     a `temperature` the probabilities of those logits are returned instead
-    (the head and the softmax in one launch where it applies)."""
+    (the softmax's statistics from the head's own launch, for a bf16 head)."""
     llama = as_llama(model, cache.device)
     step = cache.append(seq_ids, n_new)
     ids = input_ids.to(cache.device, non_blocking=True)

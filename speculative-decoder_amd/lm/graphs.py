@@ -1,9 +1,9 @@
 """HIP-graph replay of the fixed-shape forwards of the round loop.
 
 A speculative round runs the same few shapes again and again: the verify
-pass (B rows of k+1 tokens, ending in the output head fused with the
-softmax / one-hot) and the k draft steps (B rows of 1 token, ending in the
-same fused head, then the inverse-CDF sampler at T > 0, each step's token
+pass (B rows of k+1 tokens, ending in the output head, with the softmax's
+statistics, and the softmax / one-hot) and the k draft steps (B rows of 1
+token, ending in the same head, then the inverse-CDF sampler at T > 0, each step's token
 feeding the next step).  Each is captured once per
 (cache, batch, width, temperature, context bucket) and replayed; block
 allocation and the per-step metadata stay on the host side of the replay
@@ -77,7 +77,6 @@ class _Captured:
         self.llama, self.batch, self.bucket = llama, batch, bucket
         dev = cache.device
         self.ws = ops.AttentionWorkspace(dev)
-        ops.head_workspace(dev)  # allocated (and zeroed) once, outside any capture
         cfg = llama.config
         self.split = (ops.latency_split(batch, width, cfg.num_attention_heads, cfg.num_key_value_heads, bucket)
                       if latency else 0)

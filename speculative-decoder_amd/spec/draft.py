@@ -1,8 +1,8 @@
 """Drafters (reference: spec/draft.py).
 
 ModelDraft keeps the whole k-step draft loop on the GPU: each step's
-probabilities come from the output head fused with the softmax (the token
-itself from the same launch at temperature 0), its token from the inverse-CDF
+probabilities come from the output head and the softmax finished in place
+(the token itself with them at temperature 0), its token from the inverse-CDF
 kernel with a uniform drawn from the caller's generator (the reference's
 stream and order, spec/draft.py:27-29), and the sampled ids feed the next
 step's forward directly, with no host round trip between steps.

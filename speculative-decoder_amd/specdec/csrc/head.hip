@@ -1,5 +1,7 @@
 // Output head on gfx950 MFMA, with the temperature softmax / argmax of the
-// logits fused into the same launch.
+// logits: in the same launch (specdec_head_probabilities), or from statistics
+// that the head's launch leaves for a second one (specdec_head_softmax, the
+// faster at every row count).
 //
 // Reference semantics: lm/forward.py:71-84 (the final hidden rows times the
 // output head, accumulated and returned in fp32) followed by
