@@ -27,7 +27,7 @@
 // folds them per (batch, head, tile).  With 2 to 4 splits one 16-wave
 // workgroup per tile runs all of them and folds them in LDS with the same
 // arithmetic, so short contexts (decode, the draft) need one launch.  So
-// does a tiled call (5 to 12 splits, a tile for every CU): one 16-wave
+// does a tiled call (5 to 12 splits, one to four tiles for every CU): one 16-wave
 // workgroup per tile whose four wave groups take its splits in rounds,
 // every wave keeping each split's softmax state in LDS with no barrier
 // until the last; the fold then follows the split kernel's and the combine
@@ -1952,7 +1952,7 @@ struct AttnPlan {
 
 static int plan_attention(AttnArgs &a, AttnPlan &plan, int dtype, int32_t batch, int32_t width, int32_t n_heads,
                           int32_t n_kv_heads, int32_t head_dim, int32_t block_size, int32_t max_kv_len,
-                          int32_t split_tokens) {
+                          int32_t split_tokens, int64_t scratch) {
   if (batch < 0 || width < 0 || n_kv_heads <= 0 || n_heads <= 0 || n_heads % n_kv_heads ||
       block_size <= 0 || max_kv_len < 0)
     return SPECDEC_EINVAL;
@@ -1987,16 +1987,29 @@ static int plan_attention(AttnArgs &a, AttnPlan &plan, int dtype, int32_t batch,
   a.max_kv = max_kv_len;
   a.n_qtiles = qtiles(width, n_heads, n_kv_heads);
   const int64_t units = (int64_t)batch * n_kv_heads * a.n_qtiles;
-  // bf16 tiles with more than four splits (at most kTSplits), when every CU
-  // gets a tile and a tile's live rows fit kTRows, run tiled: one 16-wave
-  // workgroup per tile takes all of its splits, no partials, no combine
+  // bf16 tiles with two to four splits (or one flat split) run in one 16-wave
+  // workgroup, so that no combine launch follows.  Those with more splits (at
+  // most kTSplits), when every CU gets a tile and a tile's live rows fit
+  // kTRows, run tiled: the same with the splits in rounds.  Otherwise one
+  // 4-wave workgroup per split + combine:
+  //  - One split leaves 12 of the 16 waves idle and needs no combine either way
+  //    (5 tokens after 300, 32 heads, 16 and 4 waves: 1 row 10.4 and 9.8 us, 16
+  //    rows 23.2 and 15.0, 32 rows 43.3 and 19.7).
+  //  - A 16-wave workgroup has a compute unit to itself, so with four tiles and
+  //    more for each the workgroups' turns and the waves that ragged splits
+  //    leave idle cost more than the combine launch (32 rows after 700 / 1200 /
+  //    1900 / 2500 / 4000: 56.1 / 75.5 / 102.3 / 132.0 / 198.5 us and, combine
+  //    included, 44.8 / 67.0 / 96.1 / 122.7 / 193.9; 16 rows, two tiles for
+  //    each, after 700 / 1200 / 1900: 26.9 / 39.8 / 55.7 and 25.1 / 39.4 / 55.2,
+  //    level with the launch between).  Where the partials do not fit `scratch`
+  //    floats the one workgroup stays.
+  const int64_t cus = cu_count();
+  const bool spread = cus > 0 && units >= 4 * cus && units * a.max_splits * kPart <= scratch;
   a.tiled = dtype == SPECDEC_BF16 && !a.flat && block_size % 16 == 0 && a.max_splits > 4 &&
-            a.max_splits <= kTSplits && a.n_qtiles == 1 && width * (n_heads / n_kv_heads) <= kTRows &&
-            cu_count() > 0 && units >= cu_count();
-  // bf16 tiles with at most four splits (or one flat split, or tiled) run
-  // in one 16-wave workgroup; otherwise one 4-wave workgroup per split +
-  // combine
-  plan.single = dtype == SPECDEC_BF16 && (a.flat || a.tiled || a.max_splits <= 4);
+            a.max_splits <= kTSplits && a.n_qtiles == 1 && width * (n_heads / n_kv_heads) <= kTRows && cus > 0 &&
+            units >= cus && !spread;
+  plan.single = dtype == SPECDEC_BF16 &&
+                (a.flat || a.tiled || (a.max_splits > 1 && a.max_splits <= 4 && !spread));
   // more than kStage new tokens per row (a prompt): one pass per query tile
   plan.prefill = dtype == SPECDEC_BF16 && !a.flat && width > kStage && block_size % 16 == 0;
   if (plan.prefill) {
@@ -2092,7 +2105,7 @@ static int launch_attention(AttnArgs &a, int dtype, int32_t batch, int32_t width
                             int32_t split_tokens, float *workspace, int64_t workspace_floats, void *stream) {
   AttnPlan plan;
   const int st = plan_attention(a, plan, dtype, batch, width, n_heads, n_kv_heads, head_dim, block_size,
-                                max_kv_len, split_tokens);
+                                max_kv_len, split_tokens, workspace ? workspace_floats : 0);
   if (st != SPECDEC_OK || plan.nothing) return st;
   if (plan.need_floats > 0 && (!workspace || workspace_floats < plan.need_floats)) return SPECDEC_EINVAL;
   a.ws = workspace;
@@ -2270,7 +2283,7 @@ SPECDEC_API int specdec_paged_attention_static(const void *q, int dtype, int64_t
   a.out_stride = out_token_stride;
   AttnPlan plan;
   const int st = plan_attention(a, plan, dtype, batch, width, n_heads, n_kv_heads, head_dim, block_size,
-                                max_kv_len, split_tokens);
+                                max_kv_len, split_tokens, kStaticPartialFloats);
   if (st != SPECDEC_OK || plan.nothing) return st;
   if (plan.need_floats > kStaticPartialFloats) return SPECDEC_ENOSCRATCH;
   if (plan.need_floats > 0) {

@@ -951,3 +951,40 @@ def test_slots_past_the_keys_may_hold_anything(dtype, bs, total, t_new):
         got = out.view(n, t_new, h, d).transpose(1, 2).float().cpu()
         # fp32 sums; bf16 outputs of magnitude up to 2, p rounded to bf16
         assert (got - want).abs().max().item() < (2e-5 if dtype == torch.float32 else 2e-2), split
+
+
+@pytest.mark.parametrize("batch,length,dtype_bs", [(3, 500, 16), (40, 200, 32), (40, 200, 3), (128, 700, 16),
+                                                    (128, 2600, 16)])
+def test_short_grids_give_the_long_grids_bits(batch, length, dtype_bs):
+    """One split in four-wave workgroups, and two splits as one workgroup or
+    as two with a combine launch (four tiles for every compute unit, and no
+    workspace for the partials): the bits of each row verified alone."""
+    h = hkv = 8
+    d, bs, t = 64, dtype_bs, 5
+    g = torch.Generator(device="cuda").manual_seed(batch)
+    cache = KVCache(1, hkv, d, batch * ((length + t) // bs + 2), bs, torch.bfloat16, "cuda", max_seqs=batch)
+    ids = list(range(batch))
+    for s in ids:
+        cache.add(s)
+    total = [length + t - s % 7 for s in ids]
+    step = cache.append(ids, total)
+    k, v = (torch.randn(batch, hkv, length + t, d, generator=g, device="cuda").to(torch.bfloat16) for _ in range(2))
+    cache.write(0, step, k, v)
+    q = torch.randn(batch, t, h * d, generator=g, device="cuda").to(torch.bfloat16)
+    meta = torch.stack([step.meta[0], step.meta[2] - t, torch.full_like(step.meta[0], t)])
+
+    def call(b0, n, entry):
+        out = torch.zeros(n, t, h * d, dtype=torch.bfloat16, device="cuda")
+        x, m = q[b0:b0 + n], meta[:, b0:b0 + n].contiguous()
+        entry(x, x.stride(1), cache.k[0], cache.v[0], cache.table_tensor, m, n, t, h, hkv, d, bs, 0.125, length + t,
+              out, out.stride(1))
+        return out
+
+    together = call(0, batch, ops.paged_attention)
+    assert torch.equal(call(0, batch, ops.paged_attention_static), together)  # partials past its array: one workgroup
+    for b in (0, 1, batch // 2, batch - 1):
+        assert torch.equal(call(b, 1, ops.paged_attention)[0], together[b]), b
+    want = of.attention(q[:2].view(2, t, h, d).transpose(1, 2).float().cpu(), k[:2].float().cpu(), v[:2].float().cpu(),
+                        meta[1, :2].long().cpu(), step.meta[2, :2].long().cpu(), 0.125)
+    got = together[:2].view(2, t, h, d).transpose(1, 2).float().cpu()
+    assert (got - want).abs().max().item() < 2e-2  # bf16 outputs of magnitude up to 2, p rounded to bf16
