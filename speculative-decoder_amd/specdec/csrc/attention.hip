@@ -1392,7 +1392,7 @@ __global__ __launch_bounds__(kWave) void attention_decode_parts_kernel(AttnArgs 
 // a 16-key group are keys 8h .. 8h+7, which is the P^T operand.  One workgroup
 // of four waves per (row, kv head, 128 query rows); it walks its causal keys in
 // 64-key stages, staged into LDS once for all waves (two buffers), with the
-// loads issued two stages ahead.  The blocks with the most keys start first.
+// loads issued one stage ahead.  The blocks with the most keys start first.
 // A wave's arithmetic depends on its rows alone: a prompt's rows have the same
 // bits in any batch.  The fold order
 // differs from the split kernels', so prefill rows need not equal the bits a
@@ -1551,11 +1551,13 @@ __global__ __launch_bounds__(kPThreads) __attribute__((amdgpu_waves_per_eu(3))) 
 #pragma unroll
       for (int i = 0; i < 16; ++i) mx = fmaxf(mx, sc[kt][i]);
     mx = fmaxf(mx, other_half(mx));
-    // m, the base of the exponents, moves only when a row's maximum has left
-    // it by more than 8 (p up to 256, exact in the same way: a step that moves
-    // it rescales 32 values of O, which nearly every step did)
+    // m, the base of the exponents, is the running maximum of the row's own
+    // scores, so that the heaviest weights are rounded least (1 exactly; a
+    // base that lags by up to 2^8 grew the weights' rounding error by 6%) and
+    // a row's bits depend on no other row.  Steps in which no row of the
+    // wave has a new maximum skip the rescale, which is by 1 for the others.
     const float m_new = fmaxf(m, mx * c2);
-    if (__builtin_amdgcn_ballot_w64(m_new > m + 8.0f)) {
+    if (__builtin_amdgcn_ballot_w64(m_new > m)) {
       // (exp2(-inf) = 0 where nothing was seen before; a row with no finite
       // score yet keeps 0 as the base, so that -inf - -inf never arises)
       const float f = __builtin_amdgcn_exp2f(m - (m_new == -INFINITY ? 0.0f : m_new));

@@ -871,6 +871,66 @@ def test_prefill_rows_do_not_depend_on_the_batch_and_scales_of_any_sign():
             assert (got[b, :, :t_new[b]] - want[b, :, :t_new[b]]).abs().max().item() < 2e-2, (scale, b)
 
 
+def prompt_attention(q, k, v, past, bs=16):
+    """ops.paged_attention of one row: q [T, H, d] after `past` keys, k and v [Hkv, past + T, d]."""
+    t, h, d = q.shape
+    hkv, total = k.shape[0], past + t
+    cache = make_cache(1, hkv, d, total // bs + 4, bs, torch.bfloat16, 1)
+    cache.add(0)
+    step = cache.append([0], [total])
+    cache.write(0, step, k[None].cuda(), v[None].cuda())
+    meta = torch.tensor([[step.meta[0, 0].item()], [past], [t]], dtype=torch.int32, device="cuda")
+    out = torch.zeros(1, t, h * d, dtype=torch.bfloat16, device="cuda")
+    x = q.reshape(1, t, h * d).cuda()
+    ops.paged_attention(x, x.stride(1), cache.k[0], cache.v[0], cache.table_tensor, meta, 1, t, h, hkv, d, bs, d**-0.5,
+                        total, out, out.stride(1))
+    return out.view(t, h, d).cpu()
+
+
+@pytest.mark.parametrize("same", [9, 33])
+@pytest.mark.parametrize("heads", [(4, 4), (9, 3)])
+def test_prompt_rows_do_not_depend_on_later_tokens(same, heads):
+    """The first `same` tokens of a prompt get the same bits whatever follows
+    them: rows of the same wave with scores much larger or smaller, over keys
+    whose scores grow from step to step."""
+    h, hkv = heads
+    d, past, t = 64, 200, 50
+    g = torch.Generator().manual_seed(same)
+    q = torch.randn(t, h, d, generator=g)
+    k, v = torch.randn(hkv, past + t, d, generator=g), torch.randn(hkv, past + t, d, generator=g)
+    k *= torch.linspace(0.5, 4.0, past + t)[None, :, None]
+    k, v = k.to(torch.bfloat16), v.to(torch.bfloat16)
+    want = prompt_attention(q.to(torch.bfloat16), k, v, past)[:same]
+    for factor in (0.0, 0.1, 8.0):
+        q2, k2, v2 = q.clone(), k.clone(), v.clone()
+        q2[same:] *= factor
+        k2[:, past + same:] *= 3.0
+        v2[:, past + same:] = -v2[:, past + same:]
+        assert torch.equal(prompt_attention(q2.to(torch.bfloat16), k2, v2, past)[:same], want), factor
+
+
+def test_prompt_heaviest_weights_are_not_rounded():
+    """Two keys of nearly the same score, in two steps of the kernel, with
+    values -1 and 1: the row is the small difference of their weights, which
+    are 1 (the larger) and an fp32 rescale of 1.  Only the output's rounding to
+    bf16 (2^-9 of it) is left; weights rounded against an older base would be
+    2^-9 each, many times the difference."""
+    d, h, past, t = 64, 4, 120, 20
+    k, v = torch.zeros(h, past + t, d), torch.zeros(h, past + t, d)
+    k[:, :, 0] = -64.0
+    k[:, 3, 0], v[:, 3] = 8.0, -1.0
+    k[:, 70, 0], v[:, 70] = 8.0625, 1.0
+    q = torch.zeros(t, h, d)
+    q[:, :, 0] = torch.linspace(2.0, 20.0, t * h).view(t, h)
+    q, k, v = (x.to(torch.bfloat16) for x in (q, k, v))
+    got = prompt_attention(q, k, v, past)
+    s = q.double()[:, :, :1] * k[0].double()[None, None, :, 0] * d**-0.5  # [T, H, keys]
+    s.masked_fill_(torch.arange(past + t)[None, None, :] > past + torch.arange(t)[:, None, None], -torch.inf)
+    want = torch.softmax(s, dim=-1) @ v[0].double()
+    # 2^-9 of the output, and fp32 sums and exponents of weights near 1
+    assert ((got.double() - want).abs() <= 2.0**-8 * want.abs() + 2e-6).all()
+
+
 @pytest.mark.parametrize("lengths,heads,bs", [([31, 63, 64, 255], (4, 4), 16), ([256, 257, 507, 513], (9, 3), 48),
                                               ([769, 1020, 1, 16], (16, 1), 32)])
 def test_fp32_step_and_split_edges_match_oracle(lengths, heads, bs):
