@@ -552,6 +552,24 @@ __device__ void fold_tiled(const AttnArgs &a, const TileInfo &ti, const float *p
   store_row4<T>(a, ti, qq, d0, v);
 }
 
+// The first n (any n) of V operands' eight tokens, zeros for the others: slots
+// past a row's keys hold what a freed sequence left there, and a weight of
+// zero times an infinity or a NaN is a NaN.  g: the operand's lane group; n:
+// the keys from the chunk's first on, uniform.  (On a chunk that holds the end
+// of the keys alone, after its softmax, which runs while V is on its way;
+// chunks past it are left out.  A wave number that the compiler knows to be
+// uniform pays for the registers: 128, where scratch cost the tiled kernel 9%.)
+template <int N> __device__ __forceinline__ void keep_tokens(u32x4 (&v)[N], int g, int n) {
+  const int run = n >> 3, rem = n & 7;  // uniform: the keys end rem tokens into lane group `run`'s eight
+#pragma unroll
+  for (int w = 0; w < 4; ++w) {
+    const unsigned part = rem > 2 * w + 1 ? 0xFFFFFFFFu : rem > 2 * w ? 0xFFFFu : 0u;
+    const unsigned mask = g < run ? 0xFFFFFFFFu : g == run ? part : 0u;
+#pragma unroll
+    for (int i = 0; i < N; ++i) v[i][w] &= mask;
+  }
+}
+
 // Online-softmax update over N scores per lane (t = score * scale * log2 e,
 // -inf where not visible), replaced by their weights 2^(t - m).
 template <int N>
@@ -670,8 +688,8 @@ attention_bf16_kernel(
     return;
   }
   const bool flat = NW == 16 && a.flat;
-  const int tid = threadIdx.x, lane = tid & 63, wave = flat ? (tid >> 6) : ((tid >> 6) & 3);
-  int split_idx = (NW == 16) ? (flat ? 0 : (tid >> 8)) : (int)blockIdx.y;
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(flat ? (tid >> 6) : ((tid >> 6) & 3));
+  int split_idx = (NW == 16) ? __builtin_amdgcn_readfirstlane(flat ? 0 : (tid >> 8)) : (int)blockIdx.y;
   const int wstride = flat ? 16 * 64 : 4 * 64;  // tokens between a wave's steps
   const int g = lane >> 4, c = lane & 15;
   const int r = ti.qt * kRows + c;
@@ -1014,21 +1032,21 @@ attention_bf16_kernel(
     // reaching beyond `past`; elsewhere every score is visible
     if (c0 + 64 > ti.past) {
 #pragma unroll
-      for (int ch = 0; ch < 2; ++ch) {
+      for (int ch = 0; ch < 2; ++ch)
 #pragma unroll
         for (int j = 0; j < 8; ++j) {
           const int pos = c0 + 32 * ch + 8 * g + j;
           if (!(row_ok && pos <= qpos && pos < kv_len)) sv[8 * ch + j] = -INFINITY;
         }
-        // (a weight of zero times what a slot past the keys holds)
-        const bool live = c0 + 32 * ch + 8 * g < kv_len;
-#pragma unroll
-        for (int tt = 0; tt < 4; ++tt) r.v[ch][tt] = live ? r.v[ch][tt] : u32x4{0u, 0u, 0u, 0u};
-      }
     }
     online_update<16>(sv, m, l, o);
 #pragma unroll
     for (int ch = 0; ch < 2; ++ch) {
+      const int cs = c0 + 32 * ch;
+      if (MODE != 0 && cs + 32 > kv_len) {  // (MODE 0 loads zeros past the keys)
+        if (cs >= kv_len) break;
+        keep_tokens(r.v[ch], g, kv_len - cs);
+      }
       bf16x8 pop;
 #pragma unroll
       for (int j = 0; j < 8; ++j) pop[j] = (__bf16)sv[8 * ch + j];
@@ -1252,6 +1270,7 @@ __device__ __forceinline__ void decode_wave(const AttnArgs &a, const TileInfo &t
             r.k[ch][hf][1] = __builtin_bit_cast(u32x4, knew[1]);
           }
         }
+        keep_tokens(r.v[ch], g, kv_len - cs);  // (kv_len is p + 1)
         const int i = p - (cs + 8 * g);
         if (i >= 0 && i < 8) {
           const unsigned sh = 16 * (i & 1);
@@ -1316,7 +1335,7 @@ __global__ __launch_bounds__(kAttnThreads) __attribute__((amdgpu_waves_per_eu(2,
     AttnArgs a) {
   TileInfo ti;
   tile_coords(a, blockIdx.x, ti);
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   DecodeEarly e;
   decode_early(a, ti, lane, e);
   if (!tile_meta(a, ti, /*any_split=*/true)) {
@@ -1461,7 +1480,8 @@ __global__ __launch_bounds__(kPThreads) __attribute__((amdgpu_waves_per_eu(3))) 
   const int k_off = (x0 >> 3) * kD + (x0 & 7) * 8;        // token x0 / 8, piece x0 % 8
   const int v_dim = x0 >> 1, v_off = v_dim * bs + (x0 & 1) * 8;  // dim x0 / 2, tokens 8 (x0 % 2) ..
   // loads are unconditional (a group past the keys reads its clamped block,
-  // which is the row's own) and such groups are zeroed when stored
+  // which is the row's own); such groups, and V's slots past the keys, are
+  // zeroed when stored
   auto stage_load = [&](u32x4 (&stg)[NU], int c0, const int (&bid)[NB]) {
 #pragma unroll
     for (int i = 0; i < NB; ++i) {
@@ -1479,7 +1499,9 @@ __global__ __launch_bounds__(kPThreads) __attribute__((amdgpu_waves_per_eu(3))) 
       const int key = 16 * grp + (x0 >> 3);
       const u32x4 zero = u32x4{0u, 0u, 0u, 0u};
       *reinterpret_cast<u32x4 *>(&s_k[buf][key * kD + (((x0 & 7) ^ ((key >> 1) & 7)) * 8)]) = live ? stg[i] : zero;
-      *reinterpret_cast<u32x4 *>(&s_v[buf][grp * (16 * kD) + x0 * 8]) = live ? stg[NB + i] : zero;
+      u32x4 v[1] = {stg[NB + i]};
+      if (c0 + kPStage > wg_kv) keep_tokens(v, x0 & 1, wg_kv - (c0 + 16 * grp));
+      *reinterpret_cast<u32x4 *>(&s_v[buf][grp * (16 * kD) + x0 * 8]) = v[0];
     }
   };
 

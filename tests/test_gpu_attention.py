@@ -980,8 +980,8 @@ def test_latency_split_follows_the_keys_and_matches_the_default(batch, length, w
                                                   (torch.bfloat16, 16, [16, 528, 1040, 2064], 1)])
 def test_slots_past_the_keys_may_hold_anything(dtype, bs, total, t_new):
     """A pool of NaN but for each row's history (blocks of freed sequences hold
-    whatever those left): the fused append's rows equal the oracle's.  bf16
-    rows end at a block's end, as its kernels read whole blocks."""
+    whatever those left): the fused append's rows equal the oracle's (bf16
+    rows that end inside a block are in the next test)."""
     h, hkv, d = 4, 2, 64
     g = torch.Generator().manual_seed(bs)
     n = len(total)
@@ -1011,6 +1011,67 @@ def test_slots_past_the_keys_may_hold_anything(dtype, bs, total, t_new):
         got = out.view(n, t_new, h, d).transpose(1, 2).float().cpu()
         # fp32 sums; bf16 outputs of magnitude up to 2, p rounded to bf16
         assert (got - want).abs().max().item() < (2e-5 if dtype == torch.float32 else 2e-2), split
+
+
+@pytest.mark.parametrize("junk", [float("nan"), float("inf")])
+@pytest.mark.parametrize("bs", [16, 32, 3])
+@pytest.mark.parametrize("total,t_new", [([6, 49, 271, 530], 5), ([1, 2, 63, 65], 1), ([24, 2065, 1030, 513], 5),
+                                         ([2, 50, 271, 2048], 1), ([20, 49, 271, 530], 20),
+                                         ([200, 137, 333, 129], 129), ([4100, 37, 700, 4133], 3)])
+def test_bf16_rows_that_end_inside_a_block(total, t_new, bs, junk):
+    """The rest of a row's last block holds NaN or infinities: no row of the
+    fused append sees them, in any kernel and split (prompts past 16 tokens,
+    one-token steps, 4- and 16-wave verifies, steps left as partials)."""
+    h, hkv, d = 8, 4, 64
+    g = torch.Generator().manual_seed(bs + t_new)
+    n, longest = len(total), max(total)
+    past = [t - t_new for t in total]
+    k, v = (torch.randn(n, hkv, longest, d, generator=g).to(torch.bfloat16) for _ in range(2))
+    q = torch.randn(n, t_new, h, d, generator=g).to(torch.bfloat16)
+    qkv = torch.empty(n, t_new, (h + 2 * hkv) * d, dtype=torch.bfloat16)
+    for b in range(n):
+        new = slice(past[b], total[b])
+        qkv[b] = torch.cat([q[b].flatten(1), k[b, :, new].transpose(0, 1).flatten(1),
+                            v[b, :, new].transpose(0, 1).flatten(1)], dim=1)
+    qkv = qkv.cuda()
+    cos, sin = torch.ones(longest, d // 2, device="cuda"), torch.zeros(longest, d // 2, device="cuda")
+    want = of.attention(q.transpose(1, 2).float(), k.float(), v.float(), torch.tensor(past), torch.tensor(total), 0.125)
+
+    def fresh():
+        cache = make_cache(1, hkv, d, sum(t // bs + 2 for t in total), bs, torch.bfloat16, bs)
+        cache.k.fill_(junk)
+        cache.v.fill_(junk)
+        for s in range(n):
+            cache.add(s)
+        if max(past):
+            step = cache.append(list(range(n)), past)
+            cache.write(0, step, k[:, :, :max(past)].cuda(), v[:, :, :max(past)].cuda())
+        return cache, cache.append(list(range(n)), [t_new] * n)
+
+    def check(out):
+        got = out.view(n, t_new, h, d).transpose(1, 2).float().cpu()
+        # bf16 outputs of magnitude up to 4 (a step of 2^-6 there), p rounded to bf16
+        assert (got - want).abs().max().item() < 3e-2
+
+    for split in (0, -1, 256):
+        cache, step = fresh()
+        out = torch.zeros(n, t_new, h * d, dtype=torch.bfloat16, device="cuda")
+        ops.rope_paged_attention(qkv, cos, sin, cache.k[0], cache.v[0], cache.table_tensor, step.meta, n, t_new, h, hkv,
+                                 d, bs, 0.125, longest, out, out.stride(1), split_tokens=split)
+        check(out)
+        # the same rows, K and V already in the pool
+        if split >= 0:
+            again, x = torch.zeros_like(out), qkv[..., :h * d].contiguous()
+            ops.paged_attention(x, x.stride(1), cache.k[0], cache.v[0], cache.table_tensor, step.meta, n, t_new, h, hkv,
+                                d, bs, 0.125, longest, again, again.stride(1), split_tokens=split)
+            check(again)
+    if t_new == 1 and bs % 16 == 0:
+        cache, step = fresh()
+        parts = ops.decode_parts_buffer(n, h, qkv.device)
+        ops.rope_paged_attention_parts(qkv, cos, sin, cache.k[0], cache.v[0], cache.table_tensor, step.meta, n, h, hkv, d,
+                                       bs, 0.125, longest, parts)
+        eye = torch.eye(h * d, dtype=torch.bfloat16, device="cuda")
+        check(ops.linear_attn_parts(parts, n, h, eye, torch.zeros(n, h * d, dtype=torch.bfloat16, device="cuda")))
 
 
 @pytest.mark.parametrize("batch,length,dtype_bs", [(3, 500, 16), (40, 200, 32), (40, 200, 3), (128, 700, 16),
