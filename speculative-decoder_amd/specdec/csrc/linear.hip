@@ -574,7 +574,8 @@ __global__ __launch_bounds__(kLinMaxWaves * 64) void linear_silu_kernel(LinArgs 
 // 16-byte loads, one load instruction for four (eight) rows, written with the
 // 16-byte pieces of a row permuted by xor with its number, so that neither the writes nor
 // the operand reads meet in a bank.  The buffer is the wave's own, so no
-// barrier is needed before the fold.  The next chunk's x and W are in flight
+// barrier is needed before the fold, only an order within the wave
+// (wave_lds_order).  The next chunk's x and W are in flight
 // while one is multiplied.
 // Several feature tiles of a workgroup (NT) share a wave's x operands, which
 // halves what x costs where the weight has tiles for every compute unit
@@ -636,6 +637,16 @@ template <int Q, int NVH> struct RowScales {
   }
 };
 
+// Orders a wave's LDS accesses before and after it across the wave's lanes.
+// The hardware runs a wave's LDS operations in order, so this costs nothing
+// there; without it the compiler may move one lane's read before another
+// lane's store (it sees different addresses).
+__device__ __forceinline__ void wave_lds_order() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
 template <int NCT, int NT, int RS, typename Side>
 __device__ __forceinline__ void rows_mainloop(const LinArgs &a, const unsigned (&wbase)[NT], unsigned wstep, int row0,
                                               int lane, int s_lo, int cnt, u32x4 *s_xw, f32x4 (&acc)[NT][NCT],
@@ -681,6 +692,7 @@ __device__ __forceinline__ void rows_mainloop(const LinArgs &a, const unsigned (
       const int r = kRows * i + sub;
       s_xw[r * kPieces + (piece ^ swizzle(r))] = k.x[i];
     }
+    wave_lds_order();
 #pragma unroll
     for (int j = 0; j < RS; ++j)
 #pragma unroll
@@ -692,6 +704,7 @@ __device__ __forceinline__ void rows_mainloop(const LinArgs &a, const unsigned (
                                                                __builtin_bit_cast(bf16x8, bv), acc[t][ct], 0, 0, 0);
       }
     side.consume(k.side, b / RS);
+    wave_lds_order();  // the next stores, of a chunk or of the sums, after these reads
   };
   Chunk k0, k1;
   issue(k0, 0);
