@@ -192,7 +192,8 @@ def test_linear_silu_tiled_weight_gives_the_same_bits(rows, k, inter):
                                             (40, 160, 3000, False), (20, 96, 4112, True), (48, 288, 4112, True),
                                             (64, 2080, 4100, False), (41, 1056, 2208, True), (64, 32, 33, False),
                                             (16, 288, 4112, True), (9, 2048, 4100, False), (8, 576, 576, True),
-                                            (16, 2112, 2048, True), (17, 8192, 40, False), (20, 2112, 112, True)])
+                                            (16, 2112, 2048, True), (17, 8192, 40, False), (20, 2112, 112, True),
+                                            (64, 2048, 3072, True), (48, 2080, 3100, False)])
 def test_more_rows_equal_few_at_a_time_bitwise(rows, k, n, tiled):
     x, w = operands(rows, k, n, seed=rows + n)
     xd, wd = x.to(DEV), w.to(DEV)
@@ -212,7 +213,10 @@ def test_more_rows_equal_few_at_a_time_bitwise(rows, k, n, tiled):
                                                      (64, 160, 4800, 160, True), (20, 288, 8208, 288, True),
                                                      (40, 2048, 8208, 2048, True), (64, 544, 8200, 4096, False),
                                                      (49, 64, 104, 1024, False), (31, 2048, 1040, 4096, False),
-                                                     (16, 288, 8208, 288, True), (13, 576, 1536, 576, True)])
+                                                     (16, 288, 8208, 288, True), (13, 576, 1536, 576, True),
+                                                     (32, 2048, 5632, 2048, True), (25, 1056, 4104, 4096, False),
+                                                     (40, 2048, 3584, 1024, True), (48, 2048, 4816, 2048, True),
+                                                     (64, 2080, 4800, 4096, False)])
 def test_more_silu_rows_equal_few_at_a_time_bitwise(rows, k, inter, hdim, tiled):
     g = torch.Generator().manual_seed(rows + inter)
     w = (torch.randn(2 * inter, k, generator=g) * 0.05).to(torch.bfloat16).to(DEV)
