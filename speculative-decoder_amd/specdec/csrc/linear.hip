@@ -873,24 +873,25 @@ static void launch_linear_rows(const LinArgs &a, int64_t tiles, int waves, hipSt
 }
 
 template <int NCT, int NP, int RS, int NVH, int Q>
-static void launch_silu_rows_nvh(const LinArgs &a, int waves, const uint16_t *h, int64_t h_stride, int hd, float eps,
-                                 int inter, hipStream_t s) {
+static int launch_silu_rows_nvh(const LinArgs &a, int waves, const uint16_t *h, int64_t h_stride, int hd, float eps,
+                                int inter, hipStream_t s) {
   const dim3 grid((unsigned)(((inter + 15) / 16 + NP - 1) / NP), (unsigned)((a.M + 16 * NCT - 1) / (16 * NCT)));
   const size_t lds = (size_t)waves * kRowsLds<NCT, 2 * NP, RS> * 16;
   // more than four waves: a weight of fewer than 128 tile pairs, whose column
   // tiles are one to a workgroup (specdec_linear_silu)
   constexpr int TH = NCT == 1 && NP == 1 ? 512 : 256;
-  if (64 * waves > TH) return;  // not reached
+  if (64 * waves > TH) return SPECDEC_EUNSUPPORTED;  // (no split of today's; an error, not a call left out)
   linear_silu_rows_kernel<NCT, NP, RS, NVH, Q, TH><<<grid, 64 * waves, lds, s>>>(a, h, h_stride, hd, eps, inter);
+  return launch_status();
 }
 
 template <int NCT, int NP, int RS>
-static void launch_silu_rows(const LinArgs &a, int waves, const uint16_t *h, int64_t h_stride, int hd, float eps,
-                             int inter, hipStream_t s) {
+static int launch_silu_rows(const LinArgs &a, int waves, const uint16_t *h, int64_t h_stride, int hd, float eps,
+                            int inter, hipStream_t s) {
   const int nvec = hd / 8;
-  if (nvec <= 2 * 64) launch_silu_rows_nvh<NCT, NP, RS, 2, 3>(a, waves, h, h_stride, hd, eps, inter, s);
-  else if (nvec <= 4 * 64) launch_silu_rows_nvh<NCT, NP, RS, 4, 2>(a, waves, h, h_stride, hd, eps, inter, s);
-  else launch_silu_rows_nvh<NCT, NP, RS, 8, 1>(a, waves, h, h_stride, hd, eps, inter, s);
+  if (nvec <= 2 * 64) return launch_silu_rows_nvh<NCT, NP, RS, 2, 3>(a, waves, h, h_stride, hd, eps, inter, s);
+  if (nvec <= 4 * 64) return launch_silu_rows_nvh<NCT, NP, RS, 4, 2>(a, waves, h, h_stride, hd, eps, inter, s);
+  return launch_silu_rows_nvh<NCT, NP, RS, 8, 1>(a, waves, h, h_stride, hd, eps, inter, s);
 }
 
 // The k-split of a [N, K] weight: waves per workgroup and k-steps per wave.
@@ -1099,16 +1100,16 @@ SPECDEC_API int specdec_linear_silu(const void *x, int64_t x_stride, const void 
   const int groups = (int)std::min<int64_t>(ct, std::max<int64_t>(1, 2 * cus / tiles));
   const int nct = tiles >= 2 * cus ? ct : (ct + groups - 1) / groups;
 #define SPECDEC_SILU_ROWS(NCT, NP, RS) \
-  launch_silu_rows<NCT, NP, RS>(a, waves, h, hidden_stride, hd, eps, (int)inter, s)
+  return launch_silu_rows<NCT, NP, RS>(a, waves, h, hidden_stride, hd, eps, (int)inter, s)
   if (tiles >= 2 * cus) {
     if (nct == 1) SPECDEC_SILU_ROWS(1, 2, 2);
-    else if (nct == 2) SPECDEC_SILU_ROWS(2, 2, 2);
-    else if (nct == 3) SPECDEC_SILU_ROWS(3, 2, 2);
-    else SPECDEC_SILU_ROWS(4, 2, 2);
-  } else if (nct == 1) SPECDEC_SILU_ROWS(1, 1, 4);
-  else if (nct == 2) SPECDEC_SILU_ROWS(2, 1, 4);
-  else if (nct == 3) SPECDEC_SILU_ROWS(3, 1, 2);
-  else SPECDEC_SILU_ROWS(4, 1, 2);
+    if (nct == 2) SPECDEC_SILU_ROWS(2, 2, 2);
+    if (nct == 3) SPECDEC_SILU_ROWS(3, 2, 2);
+    SPECDEC_SILU_ROWS(4, 2, 2);
+  }
+  if (nct == 1) SPECDEC_SILU_ROWS(1, 1, 4);
+  if (nct == 2) SPECDEC_SILU_ROWS(2, 1, 4);
+  if (nct == 3) SPECDEC_SILU_ROWS(3, 1, 2);
+  SPECDEC_SILU_ROWS(4, 1, 2);
 #undef SPECDEC_SILU_ROWS
-  return launch_status();
 }
