@@ -1412,19 +1412,21 @@ __global__ __launch_bounds__(kWave) void attention_decode_parts_kernel(AttnArgs 
 // of four waves per (row, kv head, 128 query rows); it walks its causal keys in
 // 64-key stages, staged into LDS once for all waves (two buffers), with the
 // loads issued one stage ahead.  The blocks with the most keys start first.
-// A wave's arithmetic depends on its rows alone: a prompt's rows have the same
-// bits in any batch.  The fold order
-// differs from the split kernels', so prefill rows need not equal the bits a
-// decode step of the same token would get.
+// A row's arithmetic depends on the row alone: a prompt's rows have the same
+// bits in any batch that runs in the same form (KS), whatever follows them.
+// The fold order differs from the split kernels', so prefill rows need not
+// equal the bits a decode step of the same token would get.
 // MI355X, 32 heads: 4 x 1024 tokens 34 us (470 TFLOP/s), 1 x 4096 tokens 98 us
 // (700); a kernel of 16-row waves took 100 and 361.
 typedef __attribute__((ext_vector_type(16))) float f32x16;
 constexpr int kPRows = 32;                        // query rows of a wave
 constexpr int kPWaves = 4, kPThreads = kPWaves * kWave;
-constexpr int kPBlock = kPRows * kPWaves;         // query rows of a workgroup
-constexpr int kPStage = 64;                       // keys of a stage
-constexpr int kPElems = kPStage * kD;             // one stage's K, or its V
-constexpr int kPUnits = 2 * kPElems * 2 / 16 / kPThreads;  // 16-byte staging units per thread: K, then V
+// KS = 1: a wave a block of 32 rows, 64-key stages.  KS = 4: the four waves
+// share one block of 32 rows, each taking every fourth 32 keys (128-key
+// stages), and fold their (m, l, O) in LDS at the end.
+constexpr int kPShortRows = 64;  // KS = 4: calls of at most this many rows a head (run_attention has the rule)
+template <int KS> constexpr int kPBlock = kPRows * kPWaves / KS;  // query rows of a workgroup
+template <int KS> constexpr int kPStage = KS == 1 ? 64 : 128;     // keys of a stage
 
 // The lanes' other half-wave's value.
 __device__ __forceinline__ float other_half(float v) {
@@ -1432,30 +1434,32 @@ __device__ __forceinline__ float other_half(float v) {
   return __uint_as_float((threadIdx.x & 32) ? r[0] : r[1]);
 }
 
-template <int MODE>
-__global__ __launch_bounds__(kPThreads) __attribute__((amdgpu_waves_per_eu(3))) void attention_prefill_kernel(
-    AttnArgs a) {
+template <int MODE, int KS>
+__global__ __launch_bounds__(kPThreads) __attribute__((amdgpu_waves_per_eu(KS == 1 ? 3 : 2))) void
+attention_prefill_kernel(AttnArgs a) {
   typedef unsigned short u16;
-  constexpr int T = kPThreads, NU = kPUnits, NB = NU / 2;  // NB: 16-token groups a thread stages
-  __shared__ __align__(16) u16 s_k[2][kPElems];  // [key][dim], 16-byte pieces permuted by key / 2
-  __shared__ __align__(16) u16 s_v[2][kPElems];  // [16-key group][dim][16 keys]
+  constexpr int T = kPThreads, Block = kPBlock<KS>, Stage = kPStage<KS>, NKT = Stage / 32 / KS;
+  constexpr int NB = Stage * kD * 2 / 16 / T, NU = 2 * NB;  // 16-byte units a thread stages: NB of K, then NB of V
+  __shared__ __align__(16) u16 s_k[2][Stage * kD];  // [key][dim], 16-byte pieces permuted by key / 2
+  __shared__ __align__(16) u16 s_v[2][Stage * kD];  // [16-key group][dim][16 keys]
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int q = lane & 31, h = lane >> 5;
   const int Hkv = a.Hkv, group = a.H / Hkv, bhs = a.batch * Hkv;
-  const int nqb = (a.width * group + kPBlock - 1) / kPBlock;
+  const int nqb = (a.width * group + Block - 1) / Block;
   const int qb = nqb - 1 - (int)blockIdx.x / bhs, bh = (int)blockIdx.x % bhs;
   const int b = bh / Hkv, kvh = bh % Hkv;
   typedef const __attribute__((address_space(4))) int32_t const_i32;
   const_i32 *meta = (const_i32 *)a.meta;
   const int trow_i = meta[b], past = meta[a.batch + b], nrows = meta[2 * a.batch + b] * group;
-  const int r0 = qb * kPBlock;
+  const int r0 = qb * Block;
   if (r0 >= nrows) return;
   const int bs = (MODE == 1) ? 16 : a.bs;
   // no key past the call's max_kv_len is read; the rows that would need one
   // get NaN, by 16-row tiles as in the other kernels
-  const int wg_kv = min(past + (min(r0 + kPBlock, nrows) - 1) / group + 1, a.max_kv);
-  const int wr0 = r0 + kPRows * wave;
+  const int wg_kv = min(past + (min(r0 + Block, nrows) - 1) / group + 1, a.max_kv);
+  const int wr0 = KS == 1 ? r0 + kPRows * wave : r0;
+  const int k0 = KS == 1 ? 0 : 32 * wave;  // this wave's first key of a stage
   const int wave_kv = wr0 < nrows ? min(past + min(wr0 + kPRows - 1, nrows - 1) / group + 1, a.max_kv) : 0;
   const int wave_first = past + wr0 / group;  // position of the wave's first query
   const int r = min(wr0 + q, nrows - 1), t = r / group, hq = kvh * group + r % group;
@@ -1463,8 +1467,8 @@ __global__ __launch_bounds__(kPThreads) __attribute__((amdgpu_waves_per_eu(3))) 
   const bool overflow = past + min(r / kRows * kRows + kRows - 1, nrows - 1) / group + 1 > a.max_kv;
   const int qpos = min(past + t, a.max_kv - 1);  // (the bound holds for every row but those)
 
-  // ---- staging: unit tid + T i is 16 bytes of K (i < NB: 4 groups x 16
-  // tokens x 8 pieces) or of V (4 groups x 64 dims x 2); a wave's units of
+  // ---- staging: unit tid + T i is 16 bytes of K (i < NB: groups of 16
+  // tokens x 8 pieces) or of V (groups of 64 dims x 2); a wave's units of
   // one i lie in one group, so its block id is a scalar load
   const u16 *kp = reinterpret_cast<const u16 *>(a.k), *vp = reinterpret_cast<const u16 *>(a.v);
   const int64_t tile_elems = (int64_t)bs * kD;
@@ -1500,7 +1504,7 @@ __global__ __launch_bounds__(kPThreads) __attribute__((amdgpu_waves_per_eu(3))) 
       const u32x4 zero = u32x4{0u, 0u, 0u, 0u};
       *reinterpret_cast<u32x4 *>(&s_k[buf][key * kD + (((x0 & 7) ^ ((key >> 1) & 7)) * 8)]) = live ? stg[i] : zero;
       u32x4 v[1] = {stg[NB + i]};
-      if (c0 + kPStage > wg_kv) keep_tokens(v, x0 & 1, wg_kv - (c0 + 16 * grp));
+      if (c0 + Stage > wg_kv) keep_tokens(v, x0 & 1, wg_kv - (c0 + 16 * grp));
       *reinterpret_cast<u32x4 *>(&s_v[buf][grp * (16 * kD) + x0 * 8]) = v[0];
     }
   };
@@ -1544,10 +1548,10 @@ __global__ __launch_bounds__(kPThreads) __attribute__((amdgpu_waves_per_eu(3))) 
   float m = -INFINITY, l = 0.0f;  // m: the row's maximum of c2 s; l: this half-wave's part of the sum
   const int key_row = 16 * (q >> 4) + 8 * ((q >> 2) & 1) + 4 * ((q >> 3) & 1) + (q & 3);
   auto compute = [&](int c0, int buf) {
-    f32x16 sc[2];
+    f32x16 sc[NKT];
 #pragma unroll
-    for (int kt = 0; kt < 2; ++kt) {
-      const int key = 32 * kt + key_row;
+    for (int kt = 0; kt < NKT; ++kt) {
+      const int key = k0 + 32 * kt + key_row;
       f32x16 d;
 #pragma unroll
       for (int i = 0; i < 16; ++i) d[i] = 0.0f;
@@ -1558,18 +1562,18 @@ __global__ __launch_bounds__(kPThreads) __attribute__((amdgpu_waves_per_eu(3))) 
       }
       sc[kt] = d;
     }
-    if (c0 + kPStage - 1 > wave_first) {  // some key lies past some query
+    if (c0 + k0 + 32 * NKT - 1 > wave_first) {  // some key lies past some query
 #pragma unroll
-      for (int kt = 0; kt < 2; ++kt)
+      for (int kt = 0; kt < NKT; ++kt)
 #pragma unroll
         for (int i = 0; i < 16; ++i) {
-          const int pos = c0 + 32 * kt + 16 * (i >> 3) + 8 * h + (i & 7);
+          const int pos = c0 + k0 + 32 * kt + 16 * (i >> 3) + 8 * h + (i & 7);
           if (pos > qpos) sc[kt][i] = -INFINITY;
         }
     }
     float mx = sc[0][0];
 #pragma unroll
-    for (int kt = 0; kt < 2; ++kt)
+    for (int kt = 0; kt < NKT; ++kt)
 #pragma unroll
       for (int i = 0; i < 16; ++i) mx = fmaxf(mx, sc[kt][i]);
     mx = fmaxf(mx, other_half(mx));
@@ -1591,9 +1595,9 @@ __global__ __launch_bounds__(kPThreads) __attribute__((amdgpu_waves_per_eu(3))) 
       m = m_new;
     }
     const float base = m == -INFINITY ? 0.0f : m;
-    bf16x8 pop[2][2];
+    bf16x8 pop[NKT][2];
 #pragma unroll
-    for (int kt = 0; kt < 2; ++kt)
+    for (int kt = 0; kt < NKT; ++kt)
 #pragma unroll
       for (int i = 0; i < 16; ++i) {
         const float p = __builtin_amdgcn_exp2f(__builtin_fmaf(sc[kt][i], c2, -base));
@@ -1601,13 +1605,13 @@ __global__ __launch_bounds__(kPThreads) __attribute__((amdgpu_waves_per_eu(3))) 
         pop[kt][i >> 3][i & 7] = (__bf16)p;
       }
 #pragma unroll
-    for (int kt = 0; kt < 2; ++kt)
+    for (int kt = 0; kt < NKT; ++kt)
 #pragma unroll
       for (int u = 0; u < 2; ++u)
 #pragma unroll
         for (int tt = 0; tt < 2; ++tt) {
           const u32x4 vv =
-              *reinterpret_cast<const u32x4 *>(&s_v[buf][((2 * kt + u) * kD + 32 * tt + q) * 16 + 8 * h]);
+              *reinterpret_cast<const u32x4 *>(&s_v[buf][((k0 / 16 + 2 * kt + u) * kD + 32 * tt + q) * 16 + 8 * h]);
           o[tt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, vv), pop[kt][u], o[tt], 0, 0, 0);
         }
   };
@@ -1616,39 +1620,78 @@ __global__ __launch_bounds__(kPThreads) __attribute__((amdgpu_waves_per_eu(3))) 
   int bid[NB];
   blocks_of(0, bid);
   stage_load(stg, 0, bid);
-  blocks_of(kPStage, bid);
+  blocks_of(Stage, bid);
   stage_store(stg, 0, 0);
   __syncthreads();
-  for (int c0 = 0, buf = 0; c0 < wg_kv; c0 += kPStage, buf ^= 1) {
-    stage_load(stg, c0 + kPStage, bid);
-    blocks_of(c0 + 2 * kPStage, bid);
-    if (c0 < wave_kv) compute(c0, buf);
-    stage_store(stg, buf ^ 1, c0 + kPStage);
+  for (int c0 = 0, buf = 0; c0 < wg_kv; c0 += Stage, buf ^= 1) {
+    stage_load(stg, c0 + Stage, bid);
+    blocks_of(c0 + 2 * Stage, bid);
+    if (c0 + k0 < wave_kv) compute(c0, buf);
+    stage_store(stg, buf ^ 1, c0 + Stage);
     __syncthreads();
   }
-  if (!row_ok) return;
   l += other_half(l);
-  // lane (q, h) holds dims 32 tt + 8 (i / 4) + 4 h + i % 4 of its query
-  const float inv = overflow ? NAN : 1.0f / l;
   u16 *dst = reinterpret_cast<u16 *>(a.out) + ((int64_t)b * a.width + t) * a.out_stride + (int64_t)hq * kD + 4 * h;
   const bool aligned = (((uintptr_t)a.out | (uintptr_t)(a.out_stride * 2)) & 7) == 0;
+  // lane (q, h) holds dims 32 tt + 8 (i / 4) + 4 h + i % 4 of its query: run n
+  // is the four of tt = n / 4, i / 4 = n % 4
+  const float overflown = overflow ? NAN : 1.0f;
+  auto store_run = [&](int n, const float (&v)[4]) {
+    u16 w[4];
 #pragma unroll
-  for (int tt = 0; tt < 2; ++tt)
+    for (int i = 0; i < 4; ++i) w[i] = __builtin_bit_cast(u16, from_f32<__hip_bfloat16>(v[i]));
+    u16 *dd = dst + 32 * (n >> 2) + 8 * (n & 3);
+    if (aligned) {
+      *reinterpret_cast<u32x2 *>(dd) =
+          u32x2{(uint32_t)w[0] | ((uint32_t)w[1] << 16), (uint32_t)w[2] | ((uint32_t)w[3] << 16)};
+    } else {
 #pragma unroll
-    for (int i4 = 0; i4 < 4; ++i4) {
-      u16 v[4];
-#pragma unroll
-      for (int i = 0; i < 4; ++i)
-        v[i] = __builtin_bit_cast(u16, from_f32<__hip_bfloat16>(o[tt][4 * i4 + i] * inv));
-      u16 *dd = dst + 32 * tt + 8 * i4;
-      if (aligned) {
-        *reinterpret_cast<u32x2 *>(dd) =
-            u32x2{(uint32_t)v[0] | ((uint32_t)v[1] << 16), (uint32_t)v[2] | ((uint32_t)v[3] << 16)};
-      } else {
-#pragma unroll
-        for (int i = 0; i < 4; ++i) dd[i] = v[i];
-      }
+      for (int i = 0; i < 4; ++i) dd[i] = w[i];
     }
+  };
+  if constexpr (KS == 1) {
+    if (!row_ok) return;
+    const float inv = overflown / l;
+#pragma unroll
+    for (int n = 0; n < 8; ++n) {
+      const int i = 4 * (n & 3);
+      const f32x16 &ot = o[n >> 2];
+      store_run(n, {ot[i] * inv, ot[i + 1] * inv, ot[i + 2] * inv, ot[i + 3] * inv});
+    }
+  } else {
+    // the waves' states through LDS (the stages are read: the loop ended with a
+    // barrier); wave w folds and stores runs 2w and 2w + 1 of every row, the
+    // states in wave order.  A wave that saw none of a row's keys adds zeros.
+    static_assert(sizeof(s_k) >= KS * 32 * kWave * 4 && sizeof(s_v) >= KS * 2 * kWave * 4, "the states fit");
+    float *s_o = reinterpret_cast<float *>(s_k) + lane, *s_ml = reinterpret_cast<float *>(s_v) + lane;
+    s_ml[2 * wave * kWave] = m;
+    s_ml[(2 * wave + 1) * kWave] = l;
+#pragma unroll
+    for (int i = 0; i < 32; ++i) s_o[(32 * wave + i) * kWave] = o[i >> 4][i & 15];
+    __syncthreads();
+    float M = -INFINITY, L = 0.0f, f[KS];
+#pragma unroll
+    for (int w = 0; w < KS; ++w) M = fmaxf(M, s_ml[2 * w * kWave]);
+    const float base = M == -INFINITY ? 0.0f : M;
+#pragma unroll
+    for (int w = 0; w < KS; ++w) {
+      f[w] = __builtin_amdgcn_exp2f(s_ml[2 * w * kWave] - base);
+      L += f[w] * s_ml[(2 * w + 1) * kWave];
+    }
+    if (!row_ok) return;
+    const float inv = overflown / L;
+#pragma unroll
+    for (int n = 2 * wave; n < 2 * wave + 2; ++n) {
+      float v[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+      for (int w = 0; w < KS; ++w)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) v[i] += f[w] * s_o[(32 * w + 4 * n + i) * kWave];
+#pragma unroll
+      for (int i = 0; i < 4; ++i) v[i] *= inv;
+      store_run(n, v);
+    }
+  }
 }
 
 // ---------------------------------------------------------------- fp32 ----
@@ -2070,10 +2113,27 @@ static int run_attention(AttnArgs &a, const AttnPlan &plan, int dtype, int32_t b
       if (st != SPECDEC_OK) return st;
     }
     const int64_t heads = (int64_t)a.batch * a.Hkv, rows = (int64_t)a.width * (a.H / a.Hkv);
-    const int64_t blocks = heads * ((rows + kPBlock - 1) / kPBlock);
-    if (blocks > INT32_MAX || rows > INT32_MAX - kPBlock) return SPECDEC_EUNSUPPORTED;
-    if (block_size == 16) attention_prefill_kernel<1><<<(unsigned)blocks, kPThreads, 0, s>>>(a);
-    else attention_prefill_kernel<2><<<(unsigned)blocks, kPThreads, 0, s>>>(a);
+    // Up to 64 rows a head after cached keys (the next turn of a conversation) a
+    // workgroup of KS = 1 has one or two of its waves at work, and the chain of
+    // its stages is the call's time: 32 heads, 20 rows after 300 / 600 / 2000
+    // keys 10.8 / 14.9 / 34.4 us, 64 rows after 4000 65.5; KS = 4 10.4 / 12.2 /
+    // 22.6 and 39.4.  Up to 256 keys there is no chain to share and the fold is
+    // in the way (17 rows after none 7.3 and 8.7, 20 after 100 8.2 and 8.7), as
+    // it is with more workgroups than are resident at two to a compute unit
+    // (32 x 17 rows after 300: 26.3 and 28.3).
+    const bool share = rows <= kPShortRows && a.max_kv > 256 &&
+                       heads * ((rows + kPBlock<4> - 1) / kPBlock<4>) <= 2 * (int64_t)cu_count();
+    const int per = share ? kPBlock<4> : kPBlock<1>;
+    const int64_t blocks = heads * ((rows + per - 1) / per);
+    if (blocks > INT32_MAX || rows > INT32_MAX - per) return SPECDEC_EUNSUPPORTED;
+    const dim3 pgrid((unsigned)blocks), pblock(kPThreads);
+    if (share) {
+      if (block_size == 16) attention_prefill_kernel<1, 4><<<pgrid, pblock, 0, s>>>(a);
+      else attention_prefill_kernel<2, 4><<<pgrid, pblock, 0, s>>>(a);
+    } else {
+      if (block_size == 16) attention_prefill_kernel<1, 1><<<pgrid, pblock, 0, s>>>(a);
+      else attention_prefill_kernel<2, 1><<<pgrid, pblock, 0, s>>>(a);
+    }
     return launch_status();
   }
   if (plan.decode) {

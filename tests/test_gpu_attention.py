@@ -826,11 +826,16 @@ def test_short_token_buffers_are_refused_before_launch():
 
 
 # widths at the edges of the prompt kernel's 32-row waves, 128-row workgroups
-# and 64-key stages, with query heads that end a wave inside a token
+# and 64-key stages, with query heads that end a wave inside a token; up to 64
+# rows a head, four waves to 32 rows and 128-key stages, keys that end in each
+# wave's share
 @pytest.mark.parametrize("t_new,lengths,heads,bs", [(17, [1, 63], (8, 8), 16), (32, [64, 31], (4, 4), 32),
                                                     (33, [1, 200], (9, 3), 16), (43, [85, 20], (9, 3), 48),
                                                     (128, [1, 64], (4, 4), 16), (129, [300, 3], (4, 2), 16),
-                                                    (20, [700, 45], (16, 1), 16)])
+                                                    (20, [700, 45], (16, 1), 16),
+                                                    (64, [1, 127], (4, 4), 16), (65, [64, 2], (4, 4), 16),
+                                                    (21, [500, 107], (9, 3), 32), (32, [96, 65], (4, 4), 48),
+                                                    (17, [2000, 239], (4, 2), 16)])
 def test_prefill_edges_match_oracle(t_new, lengths, heads, bs):
     for got, want in run_case(2, lengths, *heads, bs, torch.bfloat16, t_new, seed=t_new):
         err = (got - want).abs()
