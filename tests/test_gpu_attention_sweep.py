@@ -94,3 +94,12 @@ def test_random_shapes_fused_append_equals_separate_kernels(batch, lengths, h, h
         outs.append((out, k_all, v_all))
     for a, b in zip(outs[0], outs[1]):
         assert torch.equal(a, b)
+
+
+# tokens at the edges of what a workgroup's threads append at once (8 tokens a
+# round, 32 with four in flight), of the 512-key splits, and past them
+@pytest.mark.parametrize("lengths,t_new,bs", [([0], 16, 16), ([5, 0], 17, 16), ([300], 32, 32), ([0, 9], 33, 16),
+                                              ([500], 70, 4), ([0], 300, 16), ([511, 40], 150, 48)])
+def test_fp32_prompts_fused_append_equals_separate_kernels(lengths, t_new, bs):
+    test_random_shapes_fused_append_equals_separate_kernels(len(lengths), lengths, 6, 2, bs, torch.float32, t_new,
+                                                            9100 + t_new)
