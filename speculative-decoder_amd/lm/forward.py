@@ -208,7 +208,7 @@ def forward(model, cache: KVCache, seq_ids: list[int], input_ids: torch.Tensor, 
                                                                                           non_blocking=True)
     cfg = llama.config
     split = (ops.latency_split(ids.shape[0], ids.shape[1], cfg.num_attention_heads, cfg.num_key_value_heads,
-                               step.max_total) if latency_split else 0)
+                               step.max_total, step.max_total) if latency_split else 0)
     return forward_core(llama, cache, step.meta, ids, step.max_total, last, split_tokens=split,
                         temperature=temperature)
 

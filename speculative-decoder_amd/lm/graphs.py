@@ -44,6 +44,14 @@ def bucket_for(max_total: int) -> int:
     return -(-max_total // BUCKET) * BUCKET
 
 
+def draft_split(llama: Llama, batch: int, width: int, bucket: int, keys: int | None = None) -> int:
+    """The attention split of a draft graph of this bucket, for rows of up to
+    `keys` keys (a batch whose best split changes inside a bucket has a graph
+    for each)."""
+    cfg = llama.config
+    return ops.latency_split(batch, width, cfg.num_attention_heads, cfg.num_key_value_heads, bucket, keys)
+
+
 def _capture(run):
     """Warm `run` up on a side stream, then capture it; returns (graph, outputs).
 
@@ -70,7 +78,7 @@ def _capture(run):
 
 class _Captured:
     def __init__(self, llama: Llama, cache: KVCache, batch: int, bucket: int, width: int,
-                 latency: bool = False) -> None:
+                 latency: bool = False, split: int | None = None) -> None:
         # the cache owns its runners (cache.graphs); a weak reference back keeps
         # that from being a cycle, so dropping a cache frees its graphs at once
         self._cache = weakref.ref(cache)
@@ -78,8 +86,9 @@ class _Captured:
         dev = cache.device
         self.ws = ops.AttentionWorkspace(dev)
         cfg = llama.config
-        self.split = (ops.latency_split(batch, width, cfg.num_attention_heads, cfg.num_key_value_heads, bucket)
-                      if latency else 0)
+        if split is None:
+            split = draft_split(llama, batch, width, bucket) if latency else 0
+        self.split = split
         self.ws.reserve(ops.attention_workspace_floats(batch, width, cfg.num_attention_heads, cfg.num_key_value_heads,
                                                        cfg.head_dim, bucket, self.split))
         self.graph = None
@@ -134,8 +143,8 @@ class DraftStepGraph(_Captured):
     """One draft step over right-padded [B, width] ids: forward of each row's
     last real token, probabilities, and an inverse-CDF sample with u[B]."""
 
-    def __init__(self, llama, cache, batch, width, temperature, bucket, latency=True):
-        super().__init__(llama, cache, batch, bucket, width, latency=latency)
+    def __init__(self, llama, cache, batch, width, temperature, bucket, latency=True, split=None):
+        super().__init__(llama, cache, batch, bucket, width, latency=latency, split=split)
         dev = cache.device
         self.temperature = temperature
         self.ids = torch.zeros(batch, width, dtype=torch.int64, device=dev)
@@ -169,8 +178,8 @@ class DraftChainGraph(_Captured):
     """`steps` consecutive one-token draft steps, each sampled token feeding
     the next step on the device.  Outputs q [B, steps, V] and tokens [B, steps]."""
 
-    def __init__(self, llama, cache, batch, steps, temperature, bucket, latency=True):
-        super().__init__(llama, cache, batch, bucket, 1, latency=latency)
+    def __init__(self, llama, cache, batch, steps, temperature, bucket, latency=True, split=None):
+        super().__init__(llama, cache, batch, bucket, 1, latency=latency, split=split)
         dev = cache.device
         self.temperature, self.steps = temperature, steps
         v = llama.config.vocab_size

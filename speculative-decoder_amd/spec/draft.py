@@ -98,11 +98,12 @@ class ModelDraft:
         u = u.to(cache.device, non_blocking=True)
         ids = torch.tensor([p + [0] * (width - len(p)) for p in pending], dtype=torch.int64)
         latency = not self.exact
-        first = graphs.get(cache, graphs.DraftStepGraph, llama, b, width, float(temperature), bucket, latency)
+        split0, split = (graphs.draft_split(llama, b, w, bucket, max_total) if latency else 0 for w in (width, 1))
+        first = graphs.get(cache, graphs.DraftStepGraph, llama, b, width, float(temperature), bucket, latency, split0)
         q0, t0 = first.run(ids, metas[0], u[0])
         if k == 1:
             return t0.clone().view(b, 1), q0.clone().view(b, 1, -1)
-        chain = graphs.get(cache, graphs.DraftChainGraph, llama, b, k - 1, float(temperature), bucket, latency)
+        chain = graphs.get(cache, graphs.DraftChainGraph, llama, b, k - 1, float(temperature), bucket, latency, split)
         qs, toks = chain.run(t0, metas[1:], u[1:])
         return torch.cat([t0.view(b, 1), toks], dim=1), torch.cat([q0.view(b, 1, -1), qs], dim=1)
 

@@ -804,21 +804,34 @@ def linear_attn_parts(parts: torch.Tensor, rows: int, n_heads: int, w: torch.Ten
     return out
 
 
-def latency_split(batch: int, width: int, n_heads: int, n_kv_heads: int, max_kv_len: int) -> int:
+def latency_split(batch: int, width: int, n_heads: int, n_kv_heads: int, max_kv_len: int,
+                  keys: int | None = None) -> int:
     """A split for calls whose bits need not match any other call (the draft
-    model).  Up to 2048 keys: -1, one workgroup per (row, head) unit striding
-    every key, so no combine kernel is launched, for one-token rows and for few
-    units, else 0 (the default).  Measured at the draft's heads, 64 rows: 7.1
-    us at 300 keys and 13.6 at 1000 against 10.3 and 14.7 with the default
-    (32 rows at 2000: 18.6 against 17.7).  Past 2048 keys one workgroup per
-    unit takes a microsecond for each 170 keys (one row of 4000: 25.6 us), so
-    the keys are split: by 256 while that gives at most four workgroups per
-    compute unit (10.9 us), else by 512 (32 rows of 2500: 18.0 against 19.9).
-    Calls of several query tiles per unit (prompts) keep -1 or 0 at any length:
-    0's splits grow with their many units, which bounds their workspace."""
-    units = batch * n_kv_heads * -(-(width * (n_heads // n_kv_heads)) // 16)
-    if max_kv_len <= 2048 or width * (n_heads // n_kv_heads) > 16:
+    model).  `keys`: the longest row's keys where max_kv_len is a bucket's.
+
+    Up to 2048 keys: -1, one workgroup per (row, head) unit striding every key,
+    so no combine kernel is launched, for few units and for one-token rows, else
+    0 (the default).  One-token rows of 64 to 192 units (22 to 64 rows of the
+    draft's heads) take the default past 1536 keys, where its fourth split
+    begins: 32 rows of 300 / 1000 / 1500 / 1600 / 2000 keys 7.1 / 11.2 / 15.1 /
+    16.8 / 18.8 us against the default's 9.8 / 12.6 / 15.8 / 15.4 / 18.0; 64 rows
+    7.1 / 14.0 / 17.9 / 19.6 / 22.1 and 9.9 / 15.2 / 18.6 / 18.4 / 21.9; at 128
+    rows -1 is ahead by 16% and more at any length.
+
+    Past 2048 keys one workgroup per unit takes a microsecond for each 170 keys
+    (one row of 4000: 25.6 us), so the keys are split: by 256 while that gives
+    at most four workgroups per compute unit (10.9 us), else by 512 (32 rows of
+    2500: 18.0 against 19.9).  Calls of several query tiles per unit (prompts)
+    keep -1 or 0 at any length: 0's splits grow with their many units, which
+    bounds their workspace."""
+    rows = width * (n_heads // n_kv_heads)
+    units = batch * n_kv_heads * -(-rows // 16)
+    if max_kv_len <= 2048:
+        if width == 1 and 64 <= units <= 192 and keys is not None and keys > 1536:
+            return 0
         return -1 if units < 64 or width == 1 else 0
+    if rows > 16:
+        return -1 if units < 64 else 0
     return 256 if units * -(-max_kv_len // 256) <= 1024 else 512
 
 

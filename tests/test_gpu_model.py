@@ -298,6 +298,47 @@ def test_graph_replay_equals_eager_launches(tiny, tiny_draft, monkeypatch, tempe
     assert runs[0] == runs[1]
 
 
+@pytest.mark.parametrize("batch,splits", [(24, {-1, 0}), (8, {-1})])
+def test_draft_graphs_follow_the_best_split_inside_a_bucket(monkeypatch, batch, splits):
+    """24 rows of 3 kv heads change their attention split at 1536 keys, inside
+    a bucket: a graph for each side, and the launches' probabilities and tokens
+    on both (fewer rows keep one graph)."""
+    from lm.model import Llama, LlamaShape
+
+    h, hq, hk, inter, v = 576, 9, 3, 256, 512
+    shape = LlamaShape(vocab_size=v, hidden_size=h, num_hidden_layers=1, num_attention_heads=hq,
+                       num_key_value_heads=hk, intermediate_size=inter, rope_theta=10000.0)
+    g = torch.Generator(device="cuda").manual_seed(batch)
+    rand = lambda *s: (torch.randn(*s, generator=g, device="cuda") * 0.05).to(torch.bfloat16)  # noqa: E731
+    p = "model.layers.0."
+    weights = {"model.embed_tokens.weight": rand(v, h), "model.norm.weight": 1 + rand(h),
+               p + "input_layernorm.weight": 1 + rand(h), p + "post_attention_layernorm.weight": 1 + rand(h),
+               p + "self_attn.q_proj.weight": rand(hq * 64, h), p + "self_attn.k_proj.weight": rand(hk * 64, h),
+               p + "self_attn.v_proj.weight": rand(hk * 64, h), p + "self_attn.o_proj.weight": rand(h, hq * 64),
+               p + "mlp.gate_proj.weight": rand(inter, h), p + "mlp.up_proj.weight": rand(inter, h),
+               p + "mlp.down_proj.weight": rand(h, inter)}
+    llama = Llama.from_state_dict(shape, weights)
+    cache = KVCache(1, hk, 64, batch * 110, 16, torch.bfloat16, "cuda", max_seqs=batch)
+    ids = list(range(batch))
+    for s in ids:
+        cache.add(s)
+    step = cache.append(ids, [1700] * batch)
+    kv = torch.randn(batch, hk, 1700, 64, generator=g, device="cuda").to(torch.bfloat16)
+    cache.write(0, step, kv, kv.flip(2))
+    drafter = ModelDraft(llama, cache)
+    for n in (1600, 1500):  # (cut back, so that both have their keys)
+        contexts = [[t % v for t in range(n + 1)]] * batch
+        outs = []
+        for flag in ("0", "1"):
+            monkeypatch.setenv("SPECDEC_GRAPHS", flag)
+            for s in ids:
+                cache.truncate(s, n)
+            outs.append(drafter.propose(ids, contexts, 3, 1.0, torch.Generator().manual_seed(n)))
+        assert torch.equal(outs[0][0], outs[1][0]) and torch.equal(outs[0][1], outs[1][1]), n
+    chains = [r for r in cache.graphs.values() if type(r).__name__ == "DraftChainGraph"]
+    assert {r.split for r in chains} == splits and len(chains) == len(splits)
+
+
 def test_graphs_are_reused_across_requests(tiny, tiny_draft, prompts, expected):
     """One cache pair serving several requests in turn: graphs captured for the
     first are replayed for the next, and outputs stay exact."""

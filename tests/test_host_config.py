@@ -48,3 +48,19 @@ def test_qwen2_is_refused():
                       num_key_value_heads=2, intermediate_size=128)
     with pytest.raises(NotImplementedError, match="qwen2"):
         shape_from_hf_config(cfg)
+
+
+@pytest.mark.parametrize("batch,heads,bucket,keys,want", [
+    # one workgroup per (row, head) wherever it is the faster: few rows, short rows, more units than compute units
+    (1, (9, 3), 2048, 2000, -1), (21, (9, 3), 2048, 2048, -1), (24, (9, 3), 2048, 300, -1),
+    (64, (9, 3), 2048, 1536, -1), (128, (9, 3), 2048, 2000, -1), (24, (9, 3), 2048, None, -1),
+    # and the default where that is: between, past its third split
+    (22, (9, 3), 2048, 1537, 0), (32, (9, 3), 2048, 2000, 0), (64, (9, 3), 1900, 1900, 0), (8, (32, 8), 2000, 2000, 0),
+    # past 2048 keys: splits, whatever the longest row has
+    (8, (9, 3), 4096, 2100, 256), (32, (9, 3), 4096, 2500, 512),
+    # more query heads to a kv head than a tile holds: 4000 keys at 64 units are too many for one workgroup each
+    (32, (32, 1), 4096, 4000, 0), (32, (32, 1), 2048, 1000, -1)])
+def test_draft_split_follows_rows_and_keys(batch, heads, bucket, keys, want):
+    from specdec import ops
+
+    assert ops.latency_split(batch, 1, *heads, bucket, keys) == want
