@@ -957,14 +957,16 @@ SPECDEC_API int specdec_linear(const void *x, int64_t x_stride, const void *w, i
     // against a workgroup a tile: 1.7B down 9.5 and 12.7 us, o 4.3 and 5.4,
     // draft down 3.3 and 3.8, draft qkv 2.78 and 2.82; with more tiles its
     // launch is too many workgroups, 1.7B qkv 8.1 and 7.7), and above it, for
-    // a long projection only, a tile in two (draft down, 9 rows: 4.1 against
-    // 3.9).
+    // a long projection only, a tile in two (1.7B down, 9 / 16 rows: 10.9 /
+    // 13.9 against 12.5 / 15.7; o from a row-major weight 5.7 / 6.7 against 6.3 /
+    // 7.4, from a tiled one 5.01 / 6.02 against 4.97 / 5.98; draft down, 9 rows:
+    // 4.1 against 3.9).
     if (rows > 8 && tiles >= cus) launch_linear_rows<1, 2, 4>(a, tiles, waves, s);
     else if (2 * tiles <= cus && rows <= 8) {
       const dim3 pg((unsigned)(2 * tiles)), pb((unsigned)(64 * ((waves + 1) / 2)));
       if (a.per_wave > 8) linear_pairs_kernel<16><<<pg, pb, 0, s>>>(a, waves);
       else linear_pairs_kernel<8><<<pg, pb, 0, s>>>(a, waves);
-    } else if (2 * tiles <= cus && a.steps >= 64)
+    } else if (2 * tiles <= cus && a.steps >= (a.w_tiled ? 65 : 64))
       linear_kernel<8, 2><<<dim3((unsigned)(2 * tiles)), block, 0, s>>>(a);
     else linear_kernel<8, 1><<<grid, block, 0, s>>>(a);
     return launch_status();
