@@ -398,8 +398,10 @@ def time_fn(fn, iters=100, graph=False):
 def bench_head():
     """The output head (49152 x 2048 target, 49152 x 576 draft, bf16) at 1 and
     5 hidden rows: torch's mm with fp32 output, that plus the softmax kernel,
-    the head kernel alone, and the head fused with the softmax.  Launches
-    cycle over copies of the head so W is read from HBM."""
+    the head kernel alone, with the row softmax, with the softmax from its own
+    statistics (head_softmax: what the forward runs) and as one launch whose
+    workgroups meet (head_fused: a library entry).  Launches cycle over copies
+    of the head so W is read from HBM."""
     from specdec import ops
 
     res = {}
@@ -423,15 +425,18 @@ def bench_head():
                  "head_logits_us": time_fn(lambda: ops.head_logits(x, w(), out=lg), graph=True),
                  "head_logits_softmax_us": time_fn(
                      lambda: ops.probabilities(ops.head_logits(x, w(), out=lg), 1.0, out=out), graph=True),
+                 "head_softmax_us": time_fn(lambda: ops.head_softmax(x, w(), 1.0, out=out), graph=True),
                  "head_fused_us": time_fn(lambda: ops.head_probabilities(x, w(), 1.0, out=out), graph=True)}
             nbytes = V * hidden * 2 + rows * hidden * 2 + rows * V * 4
             r["bytes"] = nbytes
             r["head_logits_gbs"] = nbytes / r["head_logits_us"] / 1e3
             r["head_logits_frac_of_peak"] = r["head_logits_gbs"] / HBM_PEAK_GBS
-            r["head_fused_gbs"] = nbytes / r["head_fused_us"] / 1e3
-            r["head_fused_frac_of_peak"] = r["head_fused_gbs"] / HBM_PEAK_GBS
+            for kind in ("softmax", "fused"):
+                r[f"head_{kind}_gbs"] = nbytes / r[f"head_{kind}_us"] / 1e3
+                r[f"head_{kind}_frac_of_peak"] = r[f"head_{kind}_gbs"] / HBM_PEAK_GBS
             res[f"head_{name}_rows{rows}"] = r
-            log(f"head {name} rows {rows}: logits {r['head_logits_us']:.2f} us, fused {r['head_fused_us']:.2f} us")
+            log(f"head {name} rows {rows}: logits {r['head_logits_us']:.2f} us, with the softmax "
+                f"{r['head_softmax_us']:.2f} us, one launch {r['head_fused_us']:.2f} us")
         del heads
         torch.cuda.empty_cache()
     return res
@@ -545,20 +550,23 @@ def bench_kernels(attention_grid=True):
         sets = [(tl.clone(), dl.clone()) for _ in range(copies)]
         turn = [0]
 
-        def fused_cycled():
+        def fused_cycled(temperature):
             t_, d_ = sets[turn[0] % copies]
             turn[0] += 1
-            ops.accept_reject_logits(t_, d_, 1.0, draft, ua, ur)
+            ops.accept_reject_logits(t_, d_, temperature, draft, ua, ur)
 
-        us_fused_hbm = graph_time_us(fused_cycled, per_graph=copies, replays=max(1, 2000 // copies))
+        us_fused_hbm, us_fused_hbm_t08 = (
+            graph_time_us(lambda: fused_cycled(t), per_graph=copies, replays=max(1, 2000 // copies))
+            for t in (1.0, 0.8))
         del sets
         log(f"accept b{b} k{k}: softmax {us_soft:.2f} us + accept {us_acc:.2f} us; fused {us_fused:.2f} us "
-            f"({us_fused_hbm:.2f} us with the logits from HBM)")
+            f"({us_fused_hbm:.2f} us with the logits from HBM, {us_fused_hbm_t08:.2f} at T = 0.8)")
         res[f"accept_b{b}_k{k}"] = {
             "round_bytes": logit_bytes,
             "fused_us": us_fused, "fused_gbs": logit_bytes / us_fused / 1e3,
             "fused_frac_of_peak": logit_bytes / us_fused / 1e3 / HBM_PEAK_GBS,
-            "fused_hbm_us": us_fused_hbm, "fused_hbm_frac_of_peak": logit_bytes / us_fused_hbm / 1e3 / HBM_PEAK_GBS,
+            "fused_hbm_us": us_fused_hbm, "fused_hbm_t08_us": us_fused_hbm_t08,
+            "fused_hbm_frac_of_peak": logit_bytes / us_fused_hbm / 1e3 / HBM_PEAK_GBS,
             "softmax_us": us_soft, "accept_us": us_acc, "two_launch_us": us_soft + us_acc,
             "two_launch_frac_of_peak": logit_bytes / (us_soft + us_acc) / 1e3 / HBM_PEAK_GBS,
             # what the two kernels move themselves: the softmax reads the

@@ -1,7 +1,8 @@
 // Output head on gfx950 MFMA, with the temperature softmax / argmax of the
 // logits: in the same launch (specdec_head_probabilities), or from statistics
 // that the head's launch leaves for a second one (specdec_head_softmax, the
-// faster at every row count).
+// faster at every row count, which the forward calls; the one launch is a
+// library entry for a caller that wants no second one).
 //
 // Reference semantics: lm/forward.py:71-84 (the final hidden rows times the
 // output head, accumulated and returned in fp32) followed by

@@ -482,21 +482,6 @@ def head_softmax(x: torch.Tensor, w: torch.Tensor, temperature: float, out: torc
     return o2.view(*x.shape[:-1], v) if fresh else out
 
 
-def head_fused(w: torch.Tensor, rows: int) -> bool:
-    """Whether head_probabilities takes `rows` hidden rows against head w on
-    this GPU (bf16, H a multiple of 32 up to 2048, the vocab spread over at
-    most one workgroup per compute unit with at most 16 tiles of 16 each)."""
-    if w.dtype != torch.bfloat16 or w.dim() != 2 or not (1 <= rows <= HEAD_FUSED_ROWS):
-        return False
-    v, h = w.shape
-    if h % 32 or h > 2048 or v * h * 2 > 2**31 - 1:
-        return False
-    cus = torch.cuda.get_device_properties(w.device).multi_processor_count
-    tiles = -(-v // 16)
-    tpw = max(1, -(-tiles // cus))
-    return tpw <= 16 and -(-tiles // tpw) <= min(cus, 256)
-
-
 # ------------------------------------------------------------------ n-gram --
 def ngram_lookup(history: torch.Tensor, lengths: torch.Tensor, k: int, max_n: int):
     """history int32 [B, cap], lengths int32 [B] -> (draft int64 [B, k], match int32 [B, 2])."""
