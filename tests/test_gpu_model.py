@@ -159,17 +159,18 @@ def test_identical_batched(tiny, tiny_draft, prompts, expected, batch):
         assert out == expected[i:i + batch]
 
 
-@pytest.mark.parametrize("batch,k", [(1, 4), (2, 4), (3, 4), (1, 15)])
+@pytest.mark.parametrize("batch,k", [(1, 4), (2, 4), (3, 4), (1, 15), (4, 4), (8, 4), (12, 4), (4, 15)])
 def test_bf16_identical_while_every_projection_is_row_invariant(batch, k):
-    """bf16, calls of at most 16 rows (the verify's B * (k+1) and plain
+    """bf16, calls of at most 64 rows (the verify's B * (k+1) and plain
     decoding's B): every projection runs on specdec_linear, whose rows do not
-    depend on the other rows of the call, so speculative greedy decoding
-    emits plain greedy decoding's tokens at these batches too.  (Larger
-    verify calls run on hipBLASLt, whose bits depend on the call's row
-    count; there, as on the reference's GPU path, only fp32 is exact.)"""
+    depend on the other rows of the call or on the kernel that their number
+    picks, so speculative greedy decoding emits plain greedy decoding's tokens
+    at these batches too.  (Larger verify calls run on hipBLASLt, whose bits
+    depend on the call's row count; there, as on the reference's GPU path,
+    only fp32 is exact.)"""
     model = tiny64(5, torch.bfloat16)
     draft = early_exit(model)
-    ps = random_prompts(6, model.config.vocab_size, seed=11, low=20, high=40)
+    ps = random_prompts(max(6, batch), model.config.vocab_size, seed=11, low=20, high=40)
     for i in range(0, len(ps), batch):
         chunk = ps[i:i + batch]
         want = cached_autoregressive.generate_batch(model, new_cache(model, 512, 16, torch.bfloat16), chunk, MAX_NEW)
