@@ -324,11 +324,14 @@ int specdec_attention_split(int32_t batch, int32_t width, int32_t n_heads,
  * per (row, kv head, query tile) over every key, for latency when the bits
  * need not match other calls (the draft; bf16 only, fp32 takes the default).
  * When a row needs more than four splits, a second kernel combining the
- * split partials is launched on the same stream (2 to 4 splits are folded
+ * split partials is launched on the same stream.  2 to 4 splits are folded
  * inside one workgroup with the same arithmetic, and so are 5 to 12 splits
  * when the call has a (row, kv head) tile for every compute unit and at
- * most 8 query rows per kv head: the workspace is then not used); calls
- * sharing a workspace must be ordered.  max_kv_len must bound every row's
+ * most 8 query rows per kv head: the workspace is then not used, unless the
+ * call has four tiles and more for every compute unit and a workspace that
+ * holds its partials, where the second kernel is the faster.  One split needs
+ * neither.  Calls sharing a workspace must be ordered, whatever their sizes.
+ * max_kv_len must bound every row's
  * cached length after the call (past + n_new): the grid is sized from it,
  * and a query tile whose keys pass it (16 query rows of a kv head) gets NaN
  * in its output rows (and, in the fused-append entry point, nothing

@@ -712,7 +712,8 @@ attention_bf16_kernel(
     return;
   }
   const bool flat = NW == 16 && a.flat;
-  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(flat ? (tid >> 6) : ((tid >> 6) & 3));
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(flat ? (tid >> 6) : ((tid >> 6) & 3));
   int split_idx = (NW == 16) ? __builtin_amdgcn_readfirstlane(flat ? 0 : (tid >> 8)) : (int)blockIdx.y;
   const int wstride = flat ? 16 * 64 : 4 * 64;  // tokens between a wave's steps
   const int g = lane >> 4, c = lane & 15;
@@ -2391,7 +2392,7 @@ SPECDEC_API int specdec_paged_attention_static(const void *q, int dtype, int64_t
   a.out_stride = out_token_stride;
   AttnPlan plan;
   const int st = plan_attention(a, plan, dtype, batch, width, n_heads, n_kv_heads, head_dim, block_size,
-                                max_kv_len, split_tokens, kStaticPartialFloats);
+                                max_kv_len, split_tokens, /*scratch=*/0);  // (no grid uses the array by choice)
   if (st != SPECDEC_OK || plan.nothing) return st;
   if (plan.need_floats > kStaticPartialFloats) return SPECDEC_ENOSCRATCH;
   if (plan.need_floats > 0) {

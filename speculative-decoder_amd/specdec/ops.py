@@ -677,13 +677,17 @@ def attention_workspace_floats(batch: int, width: int, n_heads: int, n_kv_heads:
     return floats.value
 
 
-_workspaces: dict[torch.device, AttentionWorkspace] = {}
+_workspaces: dict[tuple[torch.device, int], AttentionWorkspace] = {}
 
 
 def workspace_for(device: torch.device) -> AttentionWorkspace:
-    ws = _workspaces.get(device)
+    """The workspace of calls that bring none: one for each stream they are
+    made on, so that calls on two streams never share one (which calls leave
+    partials there depends on their size)."""
+    key = (device, stream())
+    ws = _workspaces.get(key)
     if ws is None:
-        ws = _workspaces[device] = AttentionWorkspace(device)
+        ws = _workspaces[key] = AttentionWorkspace(device)
     return ws
 
 

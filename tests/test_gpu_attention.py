@@ -1114,3 +1114,45 @@ def test_short_grids_give_the_long_grids_bits(batch, length, dtype_bs):
                         meta[1, :2].long().cpu(), step.meta[2, :2].long().cpu(), 0.125)
     got = together[:2].view(2, t, h, d).transpose(1, 2).float().cpu()
     assert (got - want).abs().max().item() < 2e-2  # bf16 outputs of magnitude up to 2, p rounded to bf16
+
+
+def test_calls_on_two_streams_do_not_share_the_default_workspace():
+    """Batches of four tiles a compute unit leave partials in the workspace
+    also where smaller ones leave none (at most four splits, a draft's keys
+    past 2048): calls that bring no workspace, on two streams at once, get the
+    rows that they get alone."""
+    h, d, bs, t, batch, length = 8, 64, 16, 5, 128, 700
+    g = torch.Generator(device="cuda").manual_seed(5)
+    cache = KVCache(1, h, d, batch * ((length + t) // bs + 2), bs, torch.bfloat16, "cuda", max_seqs=batch)
+    ids = list(range(batch))
+    for s in ids:
+        cache.add(s)
+    step = cache.append(ids, [length + t] * batch)
+    k, v = (torch.randn(batch, h, length + t, d, generator=g, device="cuda").to(torch.bfloat16) for _ in range(2))
+    cache.write(0, step, k, v)
+    meta = torch.stack([step.meta[0], step.meta[2] - t, torch.full_like(step.meta[0], t)])
+    qs = [torch.randn(batch, t, h * d, generator=g, device="cuda").to(torch.bfloat16) for _ in range(2)]
+
+    def call(q):
+        out = torch.empty_like(q)
+        ops.paged_attention(q, q.stride(1), cache.k[0], cache.v[0], cache.table_tensor, meta, batch, t, h, h, d, bs,
+                            0.125, length + t, out, out.stride(1))
+        return out
+
+    want = [call(q) for q in qs]
+    streams = [torch.cuda.Stream(), torch.cuda.Stream()]
+    torch.cuda.synchronize()
+    spaces = []
+    for s in streams:
+        with torch.cuda.stream(s):
+            spaces.append(ops.workspace_for(qs[0].device))
+            assert ops.workspace_for(qs[0].device) is spaces[-1]
+    assert spaces[0] is not spaces[1] and ops.workspace_for(qs[0].device) not in spaces
+    outs = [[], []]
+    for _ in range(10):
+        for i, s in enumerate(streams):
+            with torch.cuda.stream(s):
+                outs[i].append(call(qs[i]))
+    torch.cuda.synchronize()
+    for i in range(2):
+        assert all(torch.equal(out, want[i]) for out in outs[i]), i
