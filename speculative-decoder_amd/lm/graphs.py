@@ -32,7 +32,8 @@ from lm.model import Llama
 from specdec import ops
 
 # Context buckets of 2048 keys: up to four 512-token splits, which the
-# attention kernel folds inside one workgroup (no combine launch).
+# attention kernel folds inside one workgroup (no combine launch) below four
+# tiles a compute unit.  The grid is the bucket's, whatever the rows' keys.
 BUCKET = 2048
 
 

@@ -1441,8 +1441,10 @@ __global__ __launch_bounds__(kWave) void attention_decode_parts_kernel(AttnArgs 
 // bits in any batch that runs in the same form (KS), whatever follows them.
 // The fold order differs from the split kernels', so prefill rows need not
 // equal the bits a decode step of the same token would get.
-// MI355X, 32 heads: 4 x 1024 tokens 34 us (470 TFLOP/s), 1 x 4096 tokens 98 us
-// (700); a kernel of 16-row waves took 100 and 361.
+// MI355X, 32 heads, calls with RoPE and the append (graph replays): 4 x 1024
+// tokens 52.5 us, 1 x 4096 tokens 119 us; a kernel of 16-row waves took 125 and
+// 380.  In such calls this kernel takes 41.7 and 113.5 us under the tracer (605
+// TFLOP/s); 33.5 and 78 with K/V in the caches and no q to rotate.
 typedef __attribute__((ext_vector_type(16))) float f32x16;
 constexpr int kPRows = 32;                        // query rows of a wave
 constexpr int kPWaves = 4, kPThreads = kPWaves * kWave;
