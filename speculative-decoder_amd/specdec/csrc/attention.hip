@@ -1295,7 +1295,7 @@ __device__ __forceinline__ void decode_wave(const AttnArgs &a, const TileInfo &t
             r.k[ch][hf][1] = __builtin_bit_cast(u32x4, knew[1]);
           }
         }
-        keep_tokens(r.v[ch], g, kv_len - cs);  // (kv_len is p + 1)
+        if (cs + 32 > kv_len) keep_tokens(r.v[ch], g, kv_len - cs);  // (kv_len is p + 1)
         const int i = p - (cs + 8 * g);
         if (i >= 0 && i < 8) {
           const unsigned sh = 16 * (i & 1);
